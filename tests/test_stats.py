@@ -102,6 +102,34 @@ def test_groupnorm_matches_oracle(dev, pix, C):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("x_off", [0, 2])
+@pytest.mark.parametrize("C", [32, 64, 128, 256, 512])
+@pytest.mark.parametrize("pix", [1, 63, 64, 65, 129])
+def test_groupnorm_partial_rows_at_chunk_edges(dev, pix, C, x_off):
+    """Every channel count at the edges of the 64-pixel chunks, from an aligned and from a 2-byte aligned x. fp32 sums
+    of up to 64 C / 32 <= 1024 fp16 values in a tree: means within 1e-6 of the values' spread (1.5), M2 within 1e-5."""
+    print(f"gn_partial pix={pix} C={C} x_off={x_off}", flush=True)
+    rng = np.random.default_rng(pix * 31 + C)
+    x = f16(rng.standard_normal(pix * C) * 1.5 + 0.75)
+    nwg = (pix + 63) // 64
+    dx = dev.buffer(x.nbytes + 16)
+    dpart = dev.buffer((nwg + 2) * 512)
+    try:
+        dev.upload(x, dx, x_off)
+        assert dev.gn_partial(dx, pix, C, dpart, wg_off=1, x_off=x_off) == nwg
+        part = dev.read(dpart, np.float32, (nwg + 2) * 128).reshape(nwg + 2, 32, 4)
+        want = oracle.gn_partial(x, pix, C).reshape(nwg, 32, 4)
+        assert np.all(part[0] == 0) and np.all(part[-1] == 0)
+        np.testing.assert_array_equal(part[1:-1, :, 0], want[:, :, 0])
+        np.testing.assert_allclose(part[1:-1, :, 1], want[:, :, 1], rtol=1e-6, atol=1e-6)
+        np.testing.assert_allclose(part[1:-1, :, 2], want[:, :, 2], rtol=1e-5, atol=1e-5)
+        assert np.all(part[:, :, 3] == 0)
+    finally:
+        dev.free(dx)
+        dev.free(dpart)
+
+
+@pytest.mark.gpu
 def test_groupnorm_banded_partials_merge(dev):
     """gnPartial over two bands of one tensor (wgOff) then gnFinalize equals the whole-tensor statistics."""
     pix, C = 640, 128
