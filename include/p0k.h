@@ -142,7 +142,8 @@ typedef struct p0k_gn_args {
  * `heads` epilogue's layout), O [Lq][ldo] f16 with head h at column h * 128. mode 0: no mask; 1: key j visible to query
  * i iff j <= min(i, nvalid - 1); 2: j < nvalid. GQA: query head h reads kv head h / (Hq / Hkv). Zero fields take the
  * reference's defaults: Lk = Lq, Hkv = Hq, nvalid = Lk, ldo = Hq * 128, scale = 1 / sqrt(128); cap > 0 soft-caps
- * the scores to cap * tanh(s / cap). Offsets and sizes in bytes; q / k / v offsets 16-byte aligned, o 8-byte. */
+ * the scores to cap * tanh(s / cap). A call with few query rows may divide its keys over workgroups through a fixed
+ * workspace of the context (not in a capture begun by the caller, whose graph may replay on another stream). Offsets and sizes in bytes; q / k / v offsets 16-byte aligned, o 8-byte. */
 typedef struct p0k_attn_args {
   uint32_t struct_size;
   const void *q_buf; uint64_t q_off, q_size;
@@ -176,7 +177,7 @@ int p0k_ctx_create(int device, p0k_ctx **out);
 void p0k_ctx_destroy(p0k_ctx *ctx);
 int p0k_device_info_get(p0k_ctx *ctx, p0k_device_info *out);
 /* Kernel choice reads the device's CU count and the P0K_* tuning switches of the environment (P0K_MFMA_TILE,
- * P0K_MFMA_KERNEL, P0K_DMA_TAIL, P0K_GEMV_MF, P0K_GEMV_MQ4, P0K_GEMV_SLICES, P0K_ATTN_BQ) once, when the context is created;
+ * P0K_MFMA_KERNEL, P0K_DMA_TAIL, P0K_GEMV_MF, P0K_GEMV_MQ4, P0K_GEMV_SLICES, P0K_ATTN_BQ, P0K_ATTN_SPLIT) once, when the context is created;
  * p0k_ctx_reload_env reads the switches again (no counterpart in the reference, whose tuning is gpu.tune,
  * src/core/tune.js:30-36). p0k_ctx_cus: the CU count the context plans for. */
 int p0k_ctx_reload_env(p0k_ctx *ctx);

@@ -72,6 +72,7 @@ Tuning tuning_from_env(unsigned cus) {
     const int v = atoi(ov);
     if (v == 128 || v == 256) t.attn_bq = v;
   }
+  if (const char *ov = getenv("P0K_ATTN_SPLIT")) t.attn_split = atoi(ov) != 0;
   return t;
 }
 

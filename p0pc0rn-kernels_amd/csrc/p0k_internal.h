@@ -24,6 +24,7 @@ struct Tuning {
   unsigned tile_m = 0, tile_n = 0;   // P0K_MFMA_TILE=MxN
   bool dma_tail = true;        // P0K_DMA_TAIL=0: one launch for a mostly empty last round
   int attn_bq = 0;             // P0K_ATTN_BQ=128|256
+  int attn_split = -1;         // P0K_ATTN_SPLIT=0|1: attention over runs of keys never / for every call
 };
 Tuning tuning_from_env(unsigned cus);
 // validate a gemm call and translate it to kernel parameters (device pointers are filled in by the caller)

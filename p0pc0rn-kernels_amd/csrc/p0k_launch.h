@@ -51,7 +51,13 @@ struct AttnParams {
   float scale, cap;            // natural-log scale; cap > 0: scores -> cap * tanh(scores / cap)
 };
 int attention_bq(uint32_t Lq, uint32_t Hq, int cus, int force);   // queries per workgroup (force: 128 / 256 or 0)
-hipError_t launch_attention(const AttnParams &p, int cus, int force_bq, hipStream_t s);
+// the plan of a call: runs of keys (S) per kv head and 32-row block for the few-queries kernel (0: one of the
+// query-block kernels). ws: part / cnt may be used (S is at most 1 without). force: 0 / 1 (tuning), -1: the rule
+unsigned attention_runs(const AttnParams &p, int cus, bool ws, int force);
+uint64_t attention_part_bytes(int cus);       // the most the few-queries kernel leaves in `part`, and
+constexpr unsigned ATTN_COUNTERS = 1024;      // its counters (zero between calls)
+hipError_t launch_attention(const AttnParams &p, int cus, int force_bq, unsigned runs, float *part, unsigned *cnt,
+                            hipStream_t s);
 // pixstats and GroupNorm statistics (src/ops/video.js:301-321, src/ops/misc.js:50-109)
 hipError_t launch_pixstats(const void *x, uint32_t V, uint32_t C, float eps, float *r, hipStream_t s);
 hipError_t launch_gn_partial(const void *x, uint32_t pix, uint32_t C, float *part, uint32_t wg_off, hipStream_t s);

@@ -62,6 +62,12 @@ struct p0k_ctx {
   // X' of the rms / lnmod prologues for the load-to-LDS GEMM (M x K fp16, grown on demand)
   void *ws_x = nullptr;
   uint64_t ws_x_bytes = 0;
+  // partial rows and counters of attention over runs of keys: a fixed size, allocated with the context
+  float *ws_attn = nullptr;
+  uint32_t *ws_attn_cnt = nullptr;
+  // p0k_graph_begin is capturing the stream (its graphs replay in order with the context's work, so calls in them may
+  // use workspaces; a capture begun by the caller may replay anywhere)
+  bool own_capture = false;
   // 256 zero bytes: the padding taps of the load-to-LDS conv3 gather read them
   void *ws_zero = nullptr;
   // workspaces replaced by larger ones while a graph captured after their allocation may still address them: freed
@@ -103,7 +109,13 @@ int p0k_ctx_create(int device, p0k_ctx **out) {
   if (e == hipSuccess) e = hipMemset(c->ws_cnt, 0, sizeof(uint32_t) * p0k_ctx::WS_COUNTERS);
   if (e == hipSuccess) e = hipMalloc(&c->ws_zero, 256);
   if (e == hipSuccess) e = hipMemset(c->ws_zero, 0, 256);
+  if (e == hipSuccess) e = hipMalloc((void **)&c->ws_attn, p0k::attention_part_bytes((int)c->tune.cus));
+  if (e == hipSuccess) e = hipMalloc((void **)&c->ws_attn_cnt, sizeof(uint32_t) * p0k::ATTN_COUNTERS);
+  if (e == hipSuccess) e = hipMemset(c->ws_attn_cnt, 0, sizeof(uint32_t) * p0k::ATTN_COUNTERS);
+  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);   // the clears are not in order with the context's stream
   if (e != hipSuccess) {
+    if (c->ws_attn) (void)hipFree(c->ws_attn);
+    if (c->ws_attn_cnt) (void)hipFree(c->ws_attn_cnt);
     if (c->ws_cnt) (void)hipFree(c->ws_cnt);
     if (c->ws_zero) (void)hipFree(c->ws_zero);
     (void)hipStreamDestroy(c->stream);
@@ -128,6 +140,8 @@ void p0k_ctx_destroy(p0k_ctx *c) {
     for (auto &b : kv.second) (void)hipFree(b.ptr);
   if (c->ws_part) (void)hipFree(c->ws_part);
   if (c->ws_x) (void)hipFree(c->ws_x);
+  if (c->ws_attn) (void)hipFree(c->ws_attn);
+  if (c->ws_attn_cnt) (void)hipFree(c->ws_attn_cnt);
   if (c->ws_zero) (void)hipFree(c->ws_zero);
   if (c->ws_cnt) (void)hipFree(c->ws_cnt);
   for (void *p : c->ws_retired) (void)hipFree(p);
@@ -394,6 +408,16 @@ static int grow_ws(p0k_ctx *c, void **buf, uint64_t *bytes, uint64_t *epoch, uin
   *buf = nb;
   *bytes = size;
   *epoch = c->graph_epoch;
+  return P0K_OK;
+}
+
+// Whether a call that could do without may use the context's workspaces: not while a caller captures the stream, whose
+// graph may replay on any stream beside the context's own work.
+static int ws_allowed(p0k_ctx *c, bool *ok) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIPCHK(hipStreamIsCapturing(c->stream, &cs), "hipStreamIsCapturing");
+  std::lock_guard<std::mutex> lk(c->mu);
+  *ok = cs == hipStreamCaptureStatusNone || c->own_capture;
   return P0K_OK;
 }
 
@@ -665,7 +689,15 @@ int p0k_attention(p0k_ctx *c, const p0k_attn_args *a) {
       (r = check_live(c, a->v_buf, a->v_size, "attention", "v")) || (r = check_live(c, a->o_buf, a->o_size, "attention", "o")))
     return r;
   HIPCHK(hipSetDevice(c->device), "hipSetDevice");
-  hipError_t e = p0k::launch_attention(p, (int)c->tune.cus, c->tune.attn_bq, c->stream);
+  p0k::Tuning tune;
+  {
+    std::lock_guard<std::mutex> lk(c->mu);
+    tune = c->tune;
+  }
+  bool ws = true;
+  if (int rr = ws_allowed(c, &ws)) return rr;
+  const unsigned runs = tune.attn_bq ? 0u : p0k::attention_runs(p, (int)tune.cus, ws, tune.attn_split);
+  hipError_t e = p0k::launch_attention(p, (int)tune.cus, tune.attn_bq, runs, c->ws_attn, c->ws_attn_cnt, c->stream);
   if (e != hipSuccess) return hip_err(e, "attention launch");
   return P0K_OK;
 }
@@ -711,13 +743,20 @@ int p0k_graph_begin(p0k_ctx *c) {
   if (!c) return set_err(P0K_E_ARG, "graph_begin: NULL context");
   HIPCHK(hipSetDevice(c->device), "hipSetDevice");
   HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
+  std::lock_guard<std::mutex> lk(c->mu);
+  c->own_capture = true;
   return P0K_OK;
 }
 int p0k_graph_end(p0k_ctx *c, p0k_graph **out) {
   if (!c || !out) return set_err(P0K_E_ARG, "graph_end: NULL argument");
   *out = nullptr;
   hipGraph_t g = nullptr;
-  HIPCHK(hipStreamEndCapture(c->stream, &g), "hipStreamEndCapture");
+  hipError_t ce = hipStreamEndCapture(c->stream, &g);
+  {
+    std::lock_guard<std::mutex> lk(c->mu);
+    c->own_capture = false;
+  }
+  HIPCHK(ce, "hipStreamEndCapture");
   {
     std::lock_guard<std::mutex> lk(c->mu);
     c->graph_epoch++;                  // the workspaces now in use may be addressed by this graph

@@ -6,6 +6,8 @@ GPU: the HIP kernel against the oracle on the reference's own cases (test/kernel
 as attnSetup at :153-157) plus ragged lengths, GQA 8:1, an offset O with ld > Hq * 128, and the soft cap.
 Tolerance (fp16 output): |got - want| <= 2^-8 * max|want| + 2^-9 |want|, and the reference's cos > 0.9995; P is
 rounded to fp16 before the P.V products, as in the reference kernels (pv16)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -118,14 +120,82 @@ def test_attention_matches_oracle(dev, c, bq, monkeypatch):
             dev.free(d)
 
 
+# The few-queries kernel (32-row blocks of a kv head's packed query heads, runs of 32-key tiles over 4 waves): rows and
+# keys at the edges of its blocks, tiles and 128-key sets, one run and several, every mask mode
+FEW = [dict(Hq=h, Hkv=k, Lq=q, Lk=n, mode=m, nvalid=v, cap=cap) for h, k, q, n, m, v, cap in [
+    (1, 1, 1, 1, 0, 1, 0), (3, 3, 1, 31, 0, 31, 0), (8, 2, 1, 32, 2, 32, 0), (8, 2, 1, 33, 2, 33, 0),
+    (4, 4, 1, 128, 2, 127, 0), (32, 8, 1, 1000, 2, 129, 0), (32, 8, 1, 1000, 2, 999, 0), (5, 1, 2, 700, 0, 700, 0),
+    (2, 2, 16, 520, 2, 517, 0), (8, 2, 8, 300, 0, 300, 0), (3, 1, 11, 385, 2, 385, 0), (8, 2, 16, 260, 2, 255, 0),
+    (2, 1, 32, 200, 1, 20, 0), (4, 2, 16, 64, 1, 64, 0), (6, 2, 100, 333, 1, 80, 0), (2, 2, 700, 700, 1, 700, 0),
+    (3, 1, 70, 1500, 0, 1500, 0), (8, 2, 1, 900, 2, 890, 1.0), (300, 300, 1, 200, 2, 180, 0)]]
+
+
 @pytest.mark.gpu
+@pytest.mark.parametrize("how", ["eager", "graph", "caller's capture"])
+@pytest.mark.parametrize("c", FEW, ids=lambda c: "Hq{Hq} Hkv{Hkv} Lq{Lq} Lk{Lk} mode{mode} nvalid{nvalid} cap{cap}".format(**c))
+def test_attention_few_queries(dev, c, how):
+    """Against the oracle with the file's fp16 tolerance; twice with the same bits (the runs merge in order, counters
+    are left at zero), replayed from the library's graph, and under a capture begun by the caller (no workspace)."""
+    print(f"few queries {how} {c}", flush=True)
+    q, k, v = setup(c, 21, 1.0 if c["cap"] else 0.5)
+    Lq, Hq = c["Lq"], c["Hq"]
+    n, ld = Lq * (Hq * 128 + 4), Hq * 128 + 4
+    bufs = [dev.upload(q), dev.upload(k), dev.upload(v), dev.buffer(n * 2)]
+    a = {"q": {"buf": bufs[0]}, "k": {"buf": bufs[1]}, "v": {"buf": bufs[2]}, "o": {"buf": bufs[3], "ld": ld}, "Lq": Lq,
+         "Lk": c["Lk"], "Hq": Hq, "Hkv": c["Hkv"], "mode": c["mode"], "nvalid": c["nvalid"], "cap": c["cap"]}
+    got = []
+    try:
+        if how == "eager":
+            for _ in range(2):
+                dev.attention(a)
+                got.append(dev.read(bufs[3], np.uint16, n))
+        elif how == "graph":
+            dev.graph_begin()
+            dev.attention(a)
+            g = dev.graph_end()
+            for _ in range(3):
+                dev.upload(np.zeros(n, np.uint16), bufs[3])
+                dev.graph_launch(g)
+                got.append(dev.read(bufs[3], np.uint16, n))
+            dev.graph_destroy(g)
+        else:
+            hip, s = C.CDLL("libamdhip64.so"), C.c_void_p(p0k.lib().p0k_ctx_stream(dev.ctx))
+            graph, exe = C.c_void_p(), C.c_void_p()
+            dev.done()
+            assert hip.hipStreamBeginCapture(s, 1) == 0          # thread-local capture mode
+            try:
+                dev.attention(a)
+            finally:
+                assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+            for _ in range(2):
+                assert hip.hipGraphLaunch(exe, s) == 0
+                got.append(dev.read(bufs[3], np.uint16, n))
+            hip.hipGraphExecDestroy(exe)
+            hip.hipGraphDestroy(graph)
+    finally:
+        for b in bufs:
+            dev.free(b)
+    assert all(np.array_equal(g, got[0]) for g in got)
+    o = got[0].reshape(Lq, ld)
+    assert np.all(o[:, Hq * 128:] == 0)
+    want = oracle.h2f(oracle.attention(q, k, v, Lq, c["Lk"], Hq, c["Hkv"], c["mode"], c["nvalid"], cap=c["cap"]))
+    err = np.abs(oracle.h2f(o[:, :Hq * 128].ravel()) - want)
+    bound = 2 ** -8 * np.abs(want).max() + 2 ** -9 * np.abs(want)
+    assert np.all(err <= bound), f"max err {err.max()} (bound {bound.max()})"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("split", ["0", "1"])
 @pytest.mark.parametrize("pattern", ["slow ramp", "fast ramp", "late spike", "falling"])
-def test_attention_moving_maximum(dev, pattern):
+def test_attention_moving_maximum(dev, pattern, split, monkeypatch):
     """Scores whose row maximum keeps moving across the 64-key tiles: the kernel keeps the subtracted maximum until a
     row's maximum outgrows it by more than 8 in the log2 domain (P up to 2^8 meanwhile) and rescales O and l when it
     moves. Every query sees s_j = g(j) + noise: a slow ramp (about 4 log2 units per tile: the maximum moves every other
     tile), a fast ramp (16 per tile: every tile), one late spike (25 units in one tile) and a falling ramp (the maximum
-    is set by the first tile and never moves); against float64 numpy with the file's fp16 tolerance."""
+    is set by the first tile and never moves); against float64 numpy with the file's fp16 tolerance. Both kernels: the
+    one over 128-query blocks (split 0) and the one over runs of keys, whose runs and waves each have their own."""
+    monkeypatch.setenv("P0K_ATTN_SPLIT", split)
     Hq, Lq, Lk, D = 2, 128, 512, 128
     j = np.arange(Lk, dtype=np.float64)
     g = {"slow ramp": 0.5 * j, "fast ramp": 2.0 * j, "late spike": np.where(j == 300, 200.0, 0.0),
