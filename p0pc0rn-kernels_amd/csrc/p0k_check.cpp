@@ -211,6 +211,8 @@ int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *e
     if (conv) {
       NEED(K <= p.ks * p.ks * p.Ci, "gemm: conv K (%u) exceeds ks*ks*Ci", K);
       FITS("x", a->x_off + (uint64_t)p.Hi * p.Wi * p.Ci * 2, xav);
+      const uint64_t npix = (uint64_t)p.Hi * p.Wi;
+      p.nvox = npix < (1ull << 32) ? (uint32_t)npix : 0xffffffffu;
       if (a->c_gn) FITS("pv", ((uint64_t)p.pvOff + p.pvStride + p.Ci) * 4, a->pv_size);
       NEED(!a->c_gn || (p.pvOff % 4 == 0 && p.pvStride % 4 == 0), "gemm: pv.off and pv.stride must be multiples of 4 floats");
     } else {
@@ -349,7 +351,7 @@ int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *e
     plan->kernel = kernel; plan->we = we; plan->xm = xm; plan->bm = 16; plan->bn = kernel == K_GEMV_SN ? 16 : narrow ? 64 : 128; plan->mx = mx; plan->narrow = narrow;
     // the load-to-LDS kernel where it applies (P0K_MFMA_KERNEL=reg keeps the register-staged one, for tests)
     if (kernel == K_MFMA && gemm_dma_ok(p, we, xm, wbytes) && !tune.mfma_reg) kernel = plan->kernel = K_MFMA_DMA;
-    if (kernel == K_MFMA_DMA) dma_tile(M, N, we, xm == P0K_X_CONV3 ? X_CONV3 : X_F16, tune.cus, &plan->bm, &plan->bn);
+    if (kernel == K_MFMA_DMA) dma_tile(M, N, we, xm == P0K_X_CONV3 ? X_CONV3 : xm == P0K_X_CONV ? X_CONV : X_F16, tune.cus, &plan->bm, &plan->bn);
     if (kernel == K_MFMA) mfma_tile(M, N, tune.cus, &plan->bm, &plan->bn);
     if ((kernel == K_MFMA || kernel == K_MFMA_DMA) && tune.tile_m) {
       // tuning / test override of the tile (P0K_MFMA_TILE=256x128); results do not depend on it

@@ -163,7 +163,8 @@ __device__ __forceinline__ void tile_order(const Params &p, uint32_t bid, uint32
   nt = in / rows;
 }
 
-// XG: X' rows (X_F16: an fp16 matrix) or the conv3 gather (X_CONV3: input voxels [vox][Ci], padding taps read Z)
+// XG: X' rows (X_F16: an fp16 matrix), the conv3 gather (X_CONV3: input voxels [vox][Ci], padding taps read Z) or the
+// 2-D convolution's (X_CONV: input pixels [pix][Ci], any square kernel, stride and padding, optionally 2x up-sampled)
 template <int WE, int XG, int TBM, int TBN, int NWV, int WGM>
 __global__ __launch_bounds__((64 * NWV))
 __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TBM, TBN, NWV, WGM>::OCC)))) void k_gemm_dma(Params p) {
@@ -175,13 +176,13 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   uint32_t mt, nt;
   tile_order(p, blockIdx.x, mt, nt);
-  const uint32_t mB = mt * TBM, nB = p.nbase + nt * TBN;
+  const uint32_t mB = (XG == X_CONV ? p.mbase : 0u) + mt * TBM, nB = p.nbase + nt * TBN;
   const uint32_t nk = p.K / DBK;
 
   // ---- per-lane DMA sources (step 0) and per-step advances; instruction t of this wave is number 4 t + wave of
   //      the stage's list (NWV t + wave)
   uint32_t src[NW];                                   // byte offsets from X' / the weights (both < 4 GiB)
-  uint32_t cv_it[XG == X_CONV3 ? T::WA : 1], cv_yx[XG == X_CONV3 ? T::WA : 1];   // conv3 row contexts
+  uint32_t cv_it[XG == X_CONV3 ? T::WA : 1], cv_yx[XG != X_F16 ? T::WA : 1];      // conv3 / conv row contexts
   uint32_t dst[NW];                                   // byte offset inside a stage
 #pragma unroll
   for (int t = 0; t < NW; t++) {
@@ -203,6 +204,11 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
         }
         cv_it[t] = itp;
         cv_yx[t] = (uint32_t)rc.b | ((uint32_t)rc.c << 16);
+        src[t] = 8 * c;
+      } else if constexpr (XG == X_CONV) {
+        // the row's first tap, signed 16 bits each
+        const RowCtx rc = row_ctx<X_CONV>(p, m);
+        cv_yx[t] = ((uint32_t)(rc.a * (int)p.stride - (int)p.padT) & 0xffffu) | ((uint32_t)(rc.b * (int)p.stride - (int)p.padL) << 16);
         src[t] = 8 * c;
       } else {
         src[t] = (m * p.ldx + p.kx0 + 8 * c) * 2u;
@@ -242,6 +248,12 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
     kt = kt < nk ? kt : nk - 1u;
     // conv3: the step's tap (uniform; Ci % 64 == 0, so a 64-k step stays inside one tap)
     uint32_t c0 = 0, kt3 = 0, ky = 0, kx = 0;
+    if constexpr (XG == X_CONV) {
+      const uint32_t kg = kt * DBK, tap = kg / p.Ci;
+      c0 = kg - tap * p.Ci;
+      ky = tap / p.ks;
+      kx = tap - ky * p.ks;
+    }
     if constexpr (XG == X_CONV3) {
       const uint32_t kg = kt * DBK, tap = kg / p.Ci, r9 = tap % 9u;
       c0 = kg - tap * p.Ci;
@@ -258,6 +270,12 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
         const bool in = (uint32_t)iy < p.Hi && (uint32_t)ix < p.Wi;
         const size_t vox = ((size_t)it * p.Hi + (uint32_t)iy) * p.Wi + (uint32_t)ix;
         dma16a(in ? p.X + (vox * p.Ci + c0) * 2 + src[t] * 2 : p.Z, m0);
+      } else if (XG == X_CONV && t < T::WA) {
+        const uint32_t up = p.flags & F_UP2 ? 1u : 0u;
+        const int iy = (int)(int16_t)(cv_yx[t] & 0xffffu) + (int)ky, ix = ((int)cv_yx[t] >> 16) + (int)kx;
+        const bool in = (uint32_t)iy < (p.Hi << up) && (uint32_t)ix < (p.Wi << up);
+        const size_t pix = (size_t)((uint32_t)iy >> up) * p.Wi + ((uint32_t)ix >> up);
+        dma16a(in ? p.X + (pix * p.Ci + c0) * 2 + src[t] * 2 : p.Z, m0);
       } else if (t < T::WA) dma16(p.X + (size_t)kt * 128u, src[t], m0);
       else if (T::WSPLIT ? t < T::WA + T::WC : NWV * t + wave < T::NIA + T::NIC) dma16(p.W + (size_t)kt * WSTEP, src[t], m0);
       else dma4(p.W + (size_t)kt * WSTEP, src[t], m0);
@@ -496,7 +514,7 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
 template <int WE, int XG, int TBM, int TBN, int NWV = 4, int WGM = 2>
 hipError_t launch_dma_one(const Params &p, hipStream_t s) {
   Params q = p;
-  q.tilesM = (p.M + TBM - 1) / TBM;
+  q.tilesM = (p.M - p.mbase + TBM - 1) / TBM;
   q.tilesN = (p.N - p.nbase + TBN - 1) / TBN;
   hipLaunchKernelGGL((k_gemm_dma<WE, XG, TBM, TBN, NWV, WGM>), dim3(q.tilesM * q.tilesN), dim3(64 * NWV), 0, s, q);
   return hipGetLastError();
@@ -545,6 +563,28 @@ __global__ __launch_bounds__(256) void k_pnprep(Params p, uint16_t *xp) {
   }
 }
 
+// 2-D convolution: GroupNorm-apply + SiLU, materialised once per input element (the fused prologue's exact fp16 values).
+// The fused form recomputes them for each of the 9 taps and each column tile, and stages through registers: GroupNorm +
+// 3x3 convolution 128 x 128 x 256 -> 256 106.8 us per pass, with this pass and the gather 55.0; 64 x 64 x 512 -> 512
+// 183 -> 76, 256 x 256 x 128 -> 128 77 -> 50.
+__global__ __launch_bounds__(256) void k_gnprep(Params p, uint16_t *xp) {
+  const uint32_t c8 = p.Ci / 8;
+  const uint64_t n = (uint64_t)p.nvox * c8;
+  for (uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (uint64_t)gridDim.x * 256) {
+    const uint64_t pix = t / c8;
+    const uint32_t c0 = (uint32_t)(t - pix * c8) * 8;
+    const u32x4 v = *(const u32x4 *)(p.X + (pix * p.Ci + c0) * 2);
+    const f32x4 *a = (const f32x4 *)(p.PV + p.pvOff + c0), *b = (const f32x4 *)(p.PV + p.pvOff + p.pvStride + c0);
+    const f32x4 a0 = a[0], a1 = a[1], b0 = b[0], b1 = b[1];
+    const f16x2 h0 = as_h2(v.x), h1 = as_h2(v.y), h2 = as_h2(v.z), h3 = as_h2(v.w);
+    *(u32x4 *)(xp + pix * p.Ci + c0) =
+        (u32x4){pack2(silu((float)h0.x * a0.x + b0.x), silu((float)h0.y * a0.y + b0.y)),
+                pack2(silu((float)h1.x * a0.z + b0.z), silu((float)h1.y * a0.w + b0.w)),
+                pack2(silu((float)h2.x * a1.x + b1.x), silu((float)h2.y * a1.y + b1.y)),
+                pack2(silu((float)h3.x * a1.z + b1.z), silu((float)h3.y * a1.w + b1.w))};
+  }
+}
+
 // X' of the rms / lnmod prologues, materialised once: Xp[m][k] = xload8 (the fused prologue's exact values); one
 // workgroup per row, 8 k per thread and step
 template <int XM>
@@ -558,8 +598,12 @@ __global__ __launch_bounds__(256) void k_xprep(Params p, uint16_t *xp) {
 }  // namespace
 
 bool gemm_dma_ok(const Params &p, int we, int xm, uint64_t wbytes) {
-  if (xm != X_F16 && xm != X_RMS && xm != X_LNMOD && xm != X_CONV3) return false;
-  if (xm == X_CONV3) {
+  if (xm == X_CONV) {
+    // 64-k steps inside one tap; first-tap coordinates in signed 16 bits
+    const uint64_t rows = p.M ? ((uint64_t)p.M - 1) / p.Wo + 1 : 0;
+    const uint64_t yspan = rows * p.stride + p.padT + p.ks, xspan = (uint64_t)p.Wo * p.stride + p.padL + p.ks;
+    if (p.Ci % 64 != 0 || yspan > 32767 || xspan > 32767 || p.Hi > 16383 || p.Wi > 16383) return false;
+  } else if (xm == X_CONV3) {
     // 64-k steps inside one tap; input frames of the three time taps packed in 10 bits; (oy, ox) in 16
     if (p.Ci % 64 != 0 || p.stride > 1024 || p.ks > 1024 || p.Ho > 65535 || p.Wo > 65535 || p.nvox == 0xffffffffu)
       return false;
@@ -578,10 +622,11 @@ bool gemm_dma_ok(const Params &p, int we, int xm, uint64_t wbytes) {
 }
 
 hipError_t launch_xprep(const Params &p, int xm, uint16_t *xp, hipStream_t s) {
-  if (xm == X_CONV3) {
+  if (xm == X_CONV3 || xm == X_CONV) {
     const uint64_t n = (uint64_t)p.nvox * (p.Ci / 8);
     const unsigned blocks = (unsigned)(n / 256 < 4096 ? (n + 255) / 256 : 4096);
-    if (n) hipLaunchKernelGGL(k_pnprep, dim3(blocks), dim3(256), 0, s, p, xp);
+    if (n && xm == X_CONV3) hipLaunchKernelGGL(k_pnprep, dim3(blocks), dim3(256), 0, s, p, xp);
+    else if (n) hipLaunchKernelGGL(k_gnprep, dim3(blocks), dim3(256), 0, s, p, xp);
     return hipGetLastError();
   }
   if (p.M == 0) return hipSuccess;
@@ -617,7 +662,7 @@ void dma_tile(uint32_t M, uint32_t N, int we, int xg, unsigned cus, unsigned *bm
   // the conv3 gather computes each row's tap address per step (f16 weights, 13 x 92 x 160 x 128 clip: 256 x 128 with
   // 8 waves 244 us, 128 x 128 (two workgroups per CU) 257, 256 x 256 382 and 128 x 256 409 with 4 waves)
   const C cg[] = {{256, 256, 0.66}, {128, 256, 0.62}, {256, 128, 1.05}, {128, 128, 1.0}};
-  const C *cand = xg == X_CONV3 ? cg : (we == W_F16 ? c16 : (we == W_Q4 ? cq4 : cq8));
+  const C *cand = xg != X_F16 ? cg : (we == W_F16 ? c16 : (we == W_Q4 ? cq4 : cq8));
   double best = -1.0;
   for (int ci = 0; ci < 4; ci++) {
     const C &c = cand[ci];
@@ -667,7 +712,7 @@ void dma_tail(uint32_t M, uint32_t N, int we, unsigned bm, unsigned bn, unsigned
 
 hipError_t launch_gemm_dma(const Params &p, int we, int xg, unsigned bm, unsigned bn, unsigned cus, bool tail,
                            hipStream_t s) {
-  if (xg != X_CONV3) {
+  if (xg == X_F16) {
     uint32_t ncut = p.N;
     unsigned bm2 = bm, bn2 = bn;
     if (tail) dma_tail(p.M, p.N, we, bm, bn, cus, &ncut, &bm2, &bn2);
@@ -687,6 +732,11 @@ hipError_t launch_gemm_dma(const Params &p, int we, int xg, unsigned bm, unsigne
     case W_F16: return launch_dma_we<W_F16, X_CONV3>(p, bm, bn, cus, s);
     }
     return hipErrorInvalidValue;
+  }
+  switch (we) {
+  case W_Q4: return launch_dma_we<W_Q4, X_CONV>(p, bm, bn, cus, s);
+  case W_Q8: return launch_dma_we<W_Q8, X_CONV>(p, bm, bn, cus, s);
+  case W_F16: return launch_dma_we<W_F16, X_CONV>(p, bm, bn, cus, s);
   }
   return hipErrorInvalidValue;
 }

@@ -503,9 +503,80 @@ struct WsSource {
     *out = c->ws_x;
     return P0K_OK;
   }
+  // the X' workspace of a call that can do with less than `need`, or without: what there is of it, null where none can
+  // be had (a caller captures the stream, nothing to grow during a capture, or no memory)
+  int xws_if(uint64_t need, void **out, uint64_t *have) {
+    *out = nullptr;
+    *have = 0;
+    if (scratch) {
+      *out = scratch + SCRATCH_WS;
+      *have = std::min<uint64_t>(need, SCRATCH_BYTES - SCRATCH_WS);
+      return P0K_OK;
+    }
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(c->stream, &cs), "hipStreamIsCapturing");
+    if (cs != hipStreamCaptureStatusNone) {
+      std::lock_guard<std::mutex> lk(c->mu);
+      if (!c->own_capture) return P0K_OK;
+      if (need > c->ws_x_bytes) {
+        *out = c->ws_x;
+        *have = c->ws_x_bytes;
+        return P0K_OK;
+      }
+    }
+    const int r = grow_ws(c, &c->ws_x, &c->ws_x_bytes, &c->ws_x_epoch, need, "prologue");
+    if (r == P0K_OK) {
+      *out = c->ws_x;
+      *have = need;
+    }
+    if (r != P0K_E_NOMEM) return r;
+    (void)hipGetLastError();      // the failed allocation is not this call's error
+    return P0K_OK;
+  }
   uint32_t *counters() { return scratch ? (uint32_t *)(scratch + SCRATCH_CNT) : c->ws_cnt; }
   const void *zero() { return scratch ? (const void *)(scratch + SCRATCH_ZERO) : c->ws_zero; }
 };
+
+// 2-D convolution with GroupNorm + SiLU on the load-to-LDS kernel: they are applied once per input element into the X'
+// workspace, and the gather reads plain fp16 pixels (the register-staged kernel applies them once per tap and column
+// tile). A workspace smaller than the image takes it in bands of output rows, each with the input rows that its taps
+// touch (the K order, and so the bits, do not change); without room for one output row, the register-staged kernel.
+static hipError_t conv_gn(const p0k::Params &p0, const p0k::Plan &plan, const p0k::Tuning &tune, WsSource &ws, int *err) {
+  p0k::Params p = p0;
+  const uint64_t line = (uint64_t)p.Wi * p.Ci * 2u;                 // bytes of an input row
+  const uint32_t rows = (p.M - 1) / p.Wo + 1, up = p.flags & p0k::F_UP2 ? 1u : 0u;
+  void *xw = nullptr;
+  uint64_t have = 0;
+  if ((*err = ws.xws_if(line * p.Hi, &xw, &have))) return hipSuccess;
+  const uint64_t lines = have / line;
+  // n output rows touch at most ((n - 1) stride + ks - 1 >> up) + 1 + up input rows
+  uint64_t band = rows;
+  if (lines < p.Hi) band = lines < 1 + up || ((lines - 1 - up) << up) + 1 < p.ks ? 0 : (((lines - 1 - up) << up) + 1 - p.ks) / p.stride + 1;
+  if (!xw || band == 0) {
+    unsigned bm, bn;
+    p0k::mfma_tile(p.M, p.N, tune.cus, &bm, &bn);
+    return p0k::launch_gemm_mfma(p, plan.we, plan.xm, bm, bn, ws.c->stream);
+  }
+  for (uint64_t y0 = 0; y0 < rows; y0 += band) {
+    const uint64_t y1 = std::min<uint64_t>(rows, y0 + band);
+    // input rows [r0, r1) of output rows [y0, y1)
+    const int64_t lo = (int64_t)(y0 * p.stride) - (int64_t)p.padT, hi = (int64_t)((y1 - 1) * p.stride + p.ks - 1) - (int64_t)p.padT;
+    const int64_t top = ((int64_t)p.Hi << up) - 1;
+    if (hi >= 0 && lo <= top) {
+      const uint64_t r0 = (uint64_t)std::max<int64_t>(lo, 0) >> up, r1 = ((uint64_t)std::min(hi, top) >> up) + 1;
+      p.X = p0.X + r0 * line;
+      p.nvox = (uint32_t)((r1 - r0) * p.Wi);
+      hipError_t e = p0k::launch_xprep(p, plan.xm, (uint16_t *)xw, ws.c->stream);
+      if (e != hipSuccess) return e;
+      p.X = (const uint8_t *)xw - r0 * line;                        // rows outside [r0, r1) are not read
+    }
+    p.mbase = (uint32_t)(y0 * p.Wo);
+    p.M = (uint32_t)std::min<uint64_t>(p0.M, y1 * p.Wo);
+    hipError_t e = p0k::launch_gemm_dma(p, plan.we, P0K_X_CONV, plan.bm, plan.bn, tune.cus, false, ws.c->stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
 
 static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
   if (!c) return set_err(P0K_E_ARG, "gemm: NULL context");
@@ -571,6 +642,14 @@ static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
       p.X = (const uint8_t *)xw;
     }
     e = p0k::launch_gemm_dma(p, plan.we, P0K_X_CONV3, plan.bm, plan.bn, tune.cus, false, c->stream);
+  } else if (plan.kernel == p0k::K_MFMA_DMA && plan.xm == P0K_X_CONV) {
+    p.Z = (const uint8_t *)ws.zero();
+    if (p.flags & p0k::F_GN) {
+      e = conv_gn(p, plan, tune, ws, &r);
+      if (r) return r;
+    } else {
+      e = p0k::launch_gemm_dma(p, plan.we, P0K_X_CONV, plan.bm, plan.bn, tune.cus, false, c->stream);
+    }
   } else if (plan.kernel == p0k::K_MFMA_DMA) {
     if (plan.xm != P0K_X_F16) {
       // the prologue once per element into the X' workspace; the GEMM then reads fp16 rows

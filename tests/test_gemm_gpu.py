@@ -7,6 +7,8 @@ the reference's cosine > 0.9995 against its fp32-weight cpuGemm, the per-element
 against the oracle, bit-identity where the reference demands it (conv3 chunks / ring), and bit-exact dequantised
 weights.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -401,6 +403,88 @@ def test_conv3_gather_every_tile(dev, enc, pn, monkeypatch):
 def test_conv2d(dev, kw):
     c = make_conv2d_case(**kw)
     assert_close(c.run_device(dev), c.run_oracle(), what=f"conv2d {kw}")
+
+
+# the load-to-LDS 2-D gather (Ci % 64 == 0): every tile, kernel sizes, strides, paddings past the image, up-sampling,
+# ragged M and N, quantised weights
+@pytest.mark.parametrize("kw", [dict(Hi=19, Wi=23, N=200), dict(Hi=33, Wi=17, stride=2, N=128, gn=True), dict(Hi=9, Wi=13, up2=True, gn=True),
+                                dict(Hi=40, Wi=9, ks=1, pad=0, Ci=192), dict(Hi=12, Wi=31, ks=5, pad=3, N=130, gn=True),
+                                dict(Hi=1, Wi=1, N=64), dict(Hi=20, Wi=20, ks=4, pad=1, up2=True, stride=3),
+                                dict(enc="q4g32a.t64", Hi=15, Wi=21, N=192, gn=True), dict(enc="q8g64s.t64", Hi=16, Wi=16, N=128)], ids=str)
+def test_conv2d_gather_every_tile(dev, kw, monkeypatch):
+    kw = dict(dict(Ci=64), **kw)
+    c = make_conv2d_case(**kw)
+    want = to_float(c.run_oracle()).astype(np.float64)
+    # assert_close's tolerance; with GroupNorm + SiLU in front, X' may round to the next fp16 where the fp32 prologue
+    # is a unit off: one such term moves the sum by its weight times 2^-10 of |X'| (|a x + b| at most)
+    tol = 2.0 ** -9 * np.abs(want) + 2.0 ** -12 * np.sqrt(np.mean(want * want))
+    if kw.get("gn"):
+        a, b = c.bufs["pv"][:kw["Ci"]], c.bufs["pv"][kw["Ci"]:]
+        tol += np.abs(c.Wt).max() * 2.0 ** -10 * (np.abs(c.X).max() * np.abs(a).max() + np.abs(b).max())
+    outs = []
+    for t in MFMA_TILES:
+        banner(f"conv2d gather tile {t} {kw}")
+        monkeypatch.setenv("P0K_MFMA_TILE", t)
+        got = c.run_device(dev)
+        assert c.kernel == "mfma_dma"
+        err = np.abs(to_float(got) - want)
+        assert np.all(err <= tol), f"conv2d gather tile {t} {kw}: max {(err / tol).max()} of the tolerance"
+        outs.append(got)
+    for o in outs[1:]:
+        assert np.array_equal(o, outs[0])
+
+
+@pytest.mark.parametrize("how,kw", [("noalloc", {}), ("noalloc", dict(stride=2)), ("noalloc", dict(up2=True)), ("graph", {}),
+                                    ("caller's capture", {})])
+def test_conv2d_groupnorm_without_its_workspace(dev, how, kw):
+    """GroupNorm + SiLU go through the X' workspace. Past the scratch array the allocation-free call takes the image in
+    bands (the same bits); a capture that would have to grow it and a caller's capture are served by the
+    register-staged kernel (within the tolerance of assert_close)."""
+    size = dict(Hi=260, Wi=1000) if how == "noalloc" else dict(Hi=24, Wi=24)
+    c = make_conv2d_case(Ci=64, N=8, gn=True, **size, **kw)
+    d = {k: dev.upload(v) for k, v in c.bufs.items()}
+    hip, s = C.CDLL("libamdhip64.so"), C.c_void_p(p0k.lib().p0k_ctx_stream(dev.ctx))
+    a, n = c.args(lambda x: d[x]), c.bufs["y"].size
+    own = p0k.Device(0) if how == "graph" else None           # a context that has no workspace yet
+    try:
+        banner(f"conv2d groupnorm without workspace: {how}")
+        dev.gemm(a)
+        want = dev.read(d["y"], np.uint16, n)
+        dev.upload(np.zeros(n, np.uint16), d["y"])
+        if how == "noalloc":
+            assert size["Hi"] * size["Wi"] * 64 * 2 > p0k.lib().p0k_gemm_noalloc_scratch_bytes()
+            dev.gemm_noalloc(a)
+            got = dev.read(d["y"], np.uint16, n)
+        elif how == "graph":
+            e = {k: own.upload(v) for k, v in c.bufs.items()}
+            own.graph_begin()
+            own.gemm(c.args(lambda x: e[x]))
+            g = own.graph_end()
+            for _ in range(2):
+                own.graph_launch(g)
+                got = own.read(e["y"], np.uint16, n)
+            own.graph_destroy(g)
+        else:
+            graph, exe = C.c_void_p(), C.c_void_p()
+            dev.done()
+            assert hip.hipStreamBeginCapture(s, 1) == 0
+            try:
+                dev.gemm(a)
+            finally:
+                assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+            assert hip.hipGraphLaunch(exe, s) == 0
+            got = dev.read(d["y"], np.uint16, n)
+            hip.hipGraphExecDestroy(exe)
+            hip.hipGraphDestroy(graph)
+    finally:
+        for b in d.values():
+            dev.free(b)
+        if own:
+            own.close()
+    if how == "noalloc":
+        assert np.array_equal(got, want)
+    assert_close(got, want, what=f"conv2d groupnorm without its workspace: {how}")
 
 
 # ------------------------------------------------------------------------------------------------ rowstats, runtime
