@@ -21,7 +21,7 @@ PROBE_SRC = os.path.join(PKG, "probe", "p0k_probe.hip")
 PROBE_LIB = os.path.join(PKG, "probe", "libp0k_probe.so")   # the benchmark's measurement kernels (bench.py only)
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["p0k_gemm_mfma.hip", "p0k_gemm_dma.hip", "p0k_gemv.hip", "p0k_rowstats.hip", "p0k_stats.hip", "p0k_attention.hip", "p0k_runtime.cpp", "p0k_check.cpp", "p0k_pack.cpp"]
+SOURCES = ["p0k_gemm_mfma.hip", "p0k_gemm_dma.hip", "p0k_gemm_dma_q4.hip", "p0k_gemm_dma_q8.hip", "p0k_gemm_dma_f16.hip", "p0k_gemv.hip", "p0k_rowstats.hip", "p0k_stats.hip", "p0k_attention.hip", "p0k_runtime.cpp", "p0k_check.cpp", "p0k_pack.cpp"]
 HIP_FLAGS = [
     "-x", "hip", "--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
     # packed fp32 instructions stay off: ordinary float code only (v_pk_*_f32 are never emitted)
