@@ -177,7 +177,7 @@ int p0k_ctx_create(int device, p0k_ctx **out);
 void p0k_ctx_destroy(p0k_ctx *ctx);
 int p0k_device_info_get(p0k_ctx *ctx, p0k_device_info *out);
 /* Kernel choice reads the device's CU count and the P0K_* tuning switches of the environment (P0K_MFMA_TILE,
- * P0K_MFMA_KERNEL, P0K_DMA_TAIL, P0K_GEMV_MF, P0K_GEMV_MQ4, P0K_GEMV_SLICES, P0K_ATTN_BQ, P0K_ATTN_SPLIT) once, when the context is created;
+ * P0K_MFMA_KERNEL, P0K_DMA_TAIL, P0K_GEMV_MF, P0K_GEMV_MQ4, P0K_GEMV_SLICES, P0K_MFMA_SPLIT, P0K_ATTN_BQ, P0K_ATTN_SPLIT) once, when the context is created;
  * p0k_ctx_reload_env reads the switches again (no counterpart in the reference, whose tuning is gpu.tune,
  * src/core/tune.js:30-36). p0k_ctx_cus: the CU count the context plans for. */
 int p0k_ctx_reload_env(p0k_ctx *ctx);
@@ -186,7 +186,7 @@ int p0k_ctx_cus(p0k_ctx *ctx);
  * counterpart in the reference, whose queue is gpu.device.queue, src/core/gpu.js:15-20). A caller may capture it into
  * a graph of its own: gemm calls enqueued under any capture keep the workspaces they use alive until the context goes. */
 void *p0k_ctx_stream(p0k_ctx *ctx);
-/* Device bytes held by the context's gemm workspaces (split-decode partials, the rms / lnmod X'), and how many
+/* Device bytes held by the context's gemm workspaces (partial sums of split decode and split prefill calls, X'), and how many
  * replaced workspaces it keeps because a graph captured after they were allocated may still address them. */
 int p0k_ctx_workspace_stats(p0k_ctx *ctx, uint64_t *live_bytes, uint64_t *retired_buffers);
 
@@ -208,7 +208,7 @@ int p0k_gemm(p0k_ctx *ctx, const p0k_gemm_args *a);            /* validate + enq
 double p0k_gemm_flops(const p0k_gemm_args *a);                 /* 2*M*N*K, the reference's return value (gemm.js:326) */
 /* p0k_gemm_noalloc: p0k_gemm that allocates nothing. No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). The
- * same kernels, with every workspace (split-decode partials and counters, the rms / lnmod / PixelNorm X', the conv3
+ * same kernels, with every workspace (partial sums and counters, the rms / lnmod / PixelNorm / GroupNorm X', the conv3
  * zero block) taken from one static device array per GPU, set up when the first context on that GPU is created.
  * A call needing more than p0k_gemm_noalloc_scratch_bytes() (31.5 MiB: e.g. X' of M * K * 2 bytes) is refused with
  * P0K_E_ARG. The first context that calls it on a GPU holds that GPU's array until the context is destroyed, and calls

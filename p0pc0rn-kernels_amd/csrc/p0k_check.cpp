@@ -61,12 +61,14 @@ Tuning tuning_from_env(unsigned cus) {
   if (const char *ov = getenv("P0K_GEMV_SN")) t.gemv_sn = atoi(ov) != 0;
   if (const char *ov = getenv("P0K_MFMA_KERNEL")) t.mfma_reg = strcmp(ov, "reg") == 0;
   if (const char *ov = getenv("P0K_MFMA_TILE")) {
-    unsigned tm = 0, tn = 0;
-    if (sscanf(ov, "%ux%u", &tm, &tn) == 2 && (tm == 128 || tm == 256) && (tn == 128 || tn == 256)) {
+    unsigned tm = 0, tn = 0, wv = 0;
+    if (sscanf(ov, "%ux%ux%u", &tm, &tn, &wv) >= 2 && dma_tile_ok(P0K_ENC_Q4G32A_T64, tm, tn, wv)) {
       t.tile_m = tm;
       t.tile_n = tn;
+      t.tile_wv = wv == 2 || wv == 4 || wv == 8 ? wv : 0;
     }
   }
+  if (const char *ov = getenv("P0K_MFMA_SPLIT")) t.split = (unsigned)std::max(0, atoi(ov));
   if (const char *ov = getenv("P0K_DMA_TAIL")) t.dma_tail = atoi(ov) != 0;
   if (const char *ov = getenv("P0K_ATTN_BQ")) {
     const int v = atoi(ov);
@@ -351,14 +353,25 @@ int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *e
     plan->kernel = kernel; plan->we = we; plan->xm = xm; plan->bm = 16; plan->bn = kernel == K_GEMV_SN ? 16 : narrow ? 64 : 128; plan->mx = mx; plan->narrow = narrow;
     // the load-to-LDS kernel where it applies (P0K_MFMA_KERNEL=reg keeps the register-staged one, for tests)
     if (kernel == K_MFMA && gemm_dma_ok(p, we, xm, wbytes) && !tune.mfma_reg) kernel = plan->kernel = K_MFMA_DMA;
-    if (kernel == K_MFMA_DMA) dma_tile(M, N, we, xm == P0K_X_CONV3 ? X_CONV3 : xm == P0K_X_CONV ? X_CONV : X_F16, tune.cus, &plan->bm, &plan->bn);
-    if (kernel == K_MFMA) mfma_tile(M, N, tune.cus, &plan->bm, &plan->bn);
-    if ((kernel == K_MFMA || kernel == K_MFMA_DMA) && tune.tile_m) {
-      // tuning / test override of the tile (P0K_MFMA_TILE=256x128); results do not depend on it
-      plan->bm = tune.tile_m;
-      plan->bn = tune.tile_n;
+    plan->S = S; plan->KS = KS; plan->wv = 0;
+    if (kernel == K_MFMA_DMA) {
+      // the X' that the call materialises (fp32 rows, GroupNorm): it shares the workspace room with the partial sums
+      const int xg = xm == P0K_X_CONV3 ? X_CONV3 : xm == P0K_X_CONV ? X_CONV : X_F16;
+      const uint64_t xbytes = xf32 ? (uint64_t)M * K * 2u : (f & F_GN) ? (uint64_t)p.nvox * p.Ci * 2u : 0u;
+      DmaPlan d;
+      dma_plan(M, N, K, we, xg, xbytes, tune.cus, &d);
+      // tuning / test override of the tile (P0K_MFMA_TILE=256x128, unsplit; results do not depend on it) and the slices
+      if (tune.tile_m && dma_tile_ok(we, tune.tile_m, tune.tile_n, tune.tile_wv)) d = DmaPlan{tune.tile_m, tune.tile_n, tune.tile_wv, 1};
+      if (tune.split && xg != X_CONV3 && d.bn == 128) {
+        d.slices = std::min(tune.split, K / 64u);
+        if (d.slices > 1 && xbytes + (uint64_t)d.slices * M * dma_ldp(N) * 4u > DMA_SPLIT_BYTES) d.slices = 1;
+      }
+      plan->bm = d.bm; plan->bn = d.bn; plan->wv = d.wv; plan->S = d.slices;
     }
-    plan->S = S; plan->KS = KS;
+    if (kernel == K_MFMA) {
+      mfma_tile(M, N, tune.cus, &plan->bm, &plan->bn);
+      if (tune.tile_m && tune.tile_m % 128 == 0) { plan->bm = tune.tile_m; plan->bn = tune.tile_n; }
+    }
   }
   return P0K_OK;
 }

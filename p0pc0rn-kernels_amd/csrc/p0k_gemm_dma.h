@@ -6,7 +6,13 @@
 // One workgroup computes a TBM x TBN tile (TBM, TBN in {128, 256}): 4 waves (2 x 2) for the smaller tiles, 8 waves
 // (2 x 4, two per SIMD, so one wave's decode and LDS reads run under the other's MFMAs) for 256 x 256 and, with f16
 // or q8 weights, 256 x 128; a wave owns (TBM/2) x (TBN/2), 128 x 64 or 128 x 32 as 32x32 v_mfma_f32_32x32x16_f16
-// blocks. K moves in steps of 64 through a ring of S LDS stages:
+// blocks. For grids of few or short tiles, 8 waves lie 1 x 4 x 2 instead: a tile of any 32 rows x 128 columns, each wave
+// over all its rows and 32 columns, the two halves of the waves on alternate 64-k steps (WK = 2: a stage is two steps),
+// whose sums meet in LDS; and K may be cut into slices over workgroups (SPLIT), whose fp32 sums k_split_epi adds in slice
+// order before the epilogue. A weight is then decoded once per workgroup (2 x 4 decodes it in both row halves), the
+// padding rows are at most 31, and a step of a short tile does not wait for LDS four times: q4 77 x 6144 x 4096 40.3 ->
+// 26.1 us unsplit, 16.8 in 4 slices (profile: 5 us of K loop, 6 of two launches' fixed cost, 5 of partial sums).
+// K moves in steps of 64 through a ring of S LDS stages:
 //   X' rows      [row][128 B], the 16-byte chunk c of row r at c ^ ((r >> 1) & 7)
 //   f16 weights  the same layout, one row per ws column
 //   q4 records   per 64-column block and 32-k record: the 64 code rows [col][16 B] as stored, and the 64 (scale, min)
@@ -39,7 +45,9 @@ constexpr int DBK = 64;
 
 // NWV waves laid out WGM x (NWV / WGM): 4 as 2 x 2, 8 as 2 x 4 (two waves per SIMD), or 4 as 1 x 4 (WGM = 1: one
 // wave per SIMD, each over all TBM rows, so a decoded weight fragment feeds TBM / 32 MFMAs)
-template <int WE, int TBM, int TBN, int NWV = 4, int WGM = 2>
+// WK = 2: the two halves of the waves take alternate 64-k steps of the same tile (their sums meet at the end), so 8 waves
+// as 1 x 4 x 2 decode every weight once where 2 x 4 decode it in both row halves
+template <int WE, int TBM, int TBN, int NWV = 4, int WGM = 2, int WK = 1>
 struct DT {
   static constexpr int NT = 64 * NWV;
   static constexpr int NBLK = TBN / 64;                                        // 64-column weight blocks
@@ -47,28 +55,31 @@ struct DT {
   // weight scale words (q8: padded to NWV with repeats of the last block's)
   static constexpr int NIA = TBM / 8;
   static constexpr int NIC = WE == W_F16 ? TBN / 8 : (WE == W_Q4 ? NBLK * 2 : NBLK * 4);
-  static constexpr int NIS = WE == W_F16 ? 0 : (WE == W_Q4 ? NBLK * 2 : NWV);
-  // the A instructions split evenly over the waves; the weight code and scale instructions together (a wave's one
-  // instruction may then be a code block for some waves and a scale block for others: q4 256 x 128 with 8 waves)
-  static_assert(NIA % NWV == 0 && (NIC + NIS) % NWV == 0, "DMA instructions per wave");
-  static constexpr bool WSPLIT = NIC % NWV == 0;                               // codes / scales on whole rounds
-  static constexpr int NW = (NIA + NIC + NIS) / NWV;                           // per wave
-  static constexpr int WA = NIA / NWV, WC = NIC / NWV;
+  static constexpr int NIS = WE == W_F16 ? 0 : (WE == W_Q4 ? NBLK * 2 : NWV / WK);
+  // the A instructions of a stage (WK steps) split evenly over the waves; the weight code and scale instructions together
+  // (a wave's one instruction may then be a code block for some waves and a scale block for others: q4 256 x 128 with 8
+  // waves)
+  static_assert(WK * NIA % NWV == 0 && WK * (NIC + NIS) % NWV == 0, "DMA instructions per wave");
+  static constexpr bool WSPLIT = WK * NIC % NWV == 0;                          // codes / scales on whole rounds
+  static constexpr int NW = WK * (NIA + NIC + NIS) / NWV;                      // per wave
+  static constexpr int WA = WK * NIA / NWV, WC = WK * NIC / NWV;
   static constexpr int A_BYTES = TBM * 128;
   static constexpr int BC_BYTES = WE == W_F16 ? TBN * 128 : (WE == W_Q4 ? NBLK * 2 * 1024 : NBLK * 4 * 1024);
   static constexpr int BS_BYTES = NIS * 256;
-  static constexpr int STAGE = A_BYTES + BC_BYTES + BS_BYTES;
+  static constexpr int STEP = A_BYTES + BC_BYTES + BS_BYTES, STAGE = WK * STEP;
   static constexpr bool TWO = NWV == 4 && WGM == 2 && 4 * STAGE <= 160 * 1024 && TBM * TBN < 256 * 256;  // two WGs per CU
   static constexpr int BUDGET = TWO ? 80 * 1024 : 160 * 1024;
-  static constexpr int S = 3 * STAGE <= BUDGET ? 3 : 2;
+    static constexpr int SMAX = WK == 1 ? 3 : 4;
+  static constexpr int S = BUDGET / STAGE < SMAX ? BUDGET / STAGE : SMAX;
+  static_assert(S >= 2, "two stages");
   // the epilogue's fp32 staging: with one workgroup per CU the whole LDS is free after the K loop, so 128 rows of the
   // full tile width (or the whole 256 x 128 tile) go through it at once; two workgroups per CU keep 128 x 128 quadrants
   static constexpr bool WIDE = !TWO;
-  static constexpr int CW = WIDE ? TBN : 128, CR = WIDE ? (TBN == 128 ? TBM : 128) : 128, CLD = CW + 4;
+  static constexpr int CW = WIDE ? TBN : 128, CR = WIDE ? (TBN == 128 ? (TBM > 256 ? TBM / 2 : TBM) : 128) : 128, CLD = CW + 4;
   static constexpr int SMEM_C = CR * CLD * 4;
   static constexpr int SMEM = S * STAGE > SMEM_C ? S * STAGE : SMEM_C;
   static_assert(SMEM <= BUDGET, "LDS budget");
-  static constexpr int WGN = NWV / WGM;                                        // waves along N
+  static constexpr int WGN = NWV / WGM / WK;                                   // waves along N
   static constexpr int WTM = TBM / WGM, WTN = TBN / WGN;                       // a wave's sub-tile
   static constexpr int BI = WTM / 32, BJ = WTN / 32;                           // 32x32 blocks per wave
   static constexpr int WGS = TWO ? 2 : 1;                                      // workgroups per CU
@@ -166,19 +177,22 @@ __device__ __forceinline__ void tile_order(const Params &p, uint32_t bid, uint32
 
 // XG: X' rows (X_F16: an fp16 matrix), the conv3 gather (X_CONV3: input voxels [vox][Ci], padding taps read Z) or the
 // 2-D convolution's (X_CONV: input pixels [pix][Ci], any square kernel, stride and padding, optionally 2x up-sampled)
-template <int WE, int XG, int TBM, int TBN, int NWV, int WGM>
+// SPLIT: a workgroup takes one of p.slices slices of K and leaves fp32 sums (k_split_epi applies the epilogue)
+template <int WE, int XG, int TBM, int TBN, int NWV, int WGM, int WK, bool SPLIT>
 __global__ __launch_bounds__((64 * NWV))
-__attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TBM, TBN, NWV, WGM>::OCC)))) void k_gemm_dma(Params p) {
-  using T = DT<WE, TBM, TBN, NWV, WGM>;
+__attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE, TBM, TBN, NWV, WGM, WK>::OCC)))) void k_gemm_dma(Params p) {
+  using T = DT<WE, TBM, TBN, NWV, WGM, WK>;
   constexpr int S = T::S, BI = T::BI, BJ = T::BJ, NW = T::NW;
   constexpr int WTM = T::WTM, WTN = T::WTN;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[T::SMEM];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   uint32_t mt, nt;
-  tile_order(p, blockIdx.x, mt, nt);
+  tile_order(p, SPLIT ? blockIdx.x % (p.tilesM * p.tilesN) : blockIdx.x, mt, nt);
   const uint32_t mB = (XG == X_CONV ? p.mbase : 0u) + mt * TBM, nB = p.nbase + nt * TBN;
-  const uint32_t nk = p.K / DBK;
+  // the slice of K of this workgroup: steps [k0, k0 + nk) (one slice: all of them)
+  const uint32_t nkt = p.K / DBK, slice = blockIdx.x / (p.tilesM * p.tilesN);
+  const uint32_t ks0 = SPLIT ? nkt * slice / p.slices : 0u, nk = SPLIT ? nkt * (slice + 1) / p.slices - ks0 : nkt;
 
   // ---- per-lane DMA sources (step 0) and per-step advances; instruction t of this wave is number 4 t + wave of
   //      the stage's list (NWV t + wave)
@@ -187,8 +201,10 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
   uint32_t dst[NW];                                   // byte offset inside a stage
 #pragma unroll
   for (int t = 0; t < NW; t++) {
-    const int q = NWV * t + wave;
-    if (t < T::WA) {                                  // X' rows 8q .. 8q+7
+    int q = NWV * t + wave;
+    if (t < T::WA) {                                  // X' rows 8q .. 8q+7 (WK = 2: of the stage's step q / NIA)
+      const int kh = WK == 1 ? 0 : q / T::NIA;
+      q -= kh * T::NIA;
       const uint32_t r = 8 * q + lane / 8, c = (lane & 7) ^ ((r >> 1) & 7);
       uint32_t m = mB + r;
       m = m < p.M ? m : p.M - 1u;
@@ -214,9 +230,11 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
       } else {
         src[t] = (m * p.ldx + p.kx0 + 8 * c) * 2u;
       }
-      dst[t] = q * 1024;
-    } else if (T::WSPLIT ? t < T::WA + T::WC : q < T::NIA + T::NIC) {
-      const int b = q - T::NIA;
+      dst[t] = kh * T::STEP + q * 1024;
+    } else if (T::WSPLIT ? t < T::WA + T::WC : q < WK * (T::NIA + T::NIC)) {
+      int b = q - WK * T::NIA;
+      const int kh = WK == 1 ? 0 : b / T::NIC;
+      b -= kh * T::NIC;
       if constexpr (WE == W_F16) {                    // weight rows of ws columns 8b .. 8b+7
         const uint32_t r = 8 * b + lane / 8, c = (lane & 7) ^ ((r >> 1) & 7);
         src[t] = (wrow(p, nB + r) * p.wG + p.wk0 + 8 * c) * 2u;
@@ -227,9 +245,11 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
         const uint32_t r = wrow(p, nB + 64 * (b >> 2) + lane);
         src[t] = ((r >> 6) * p.wG + (p.wk0 >> 6)) * 4224u + (r & 63u) * 64u + (b & 3) * 16u;
       }
-      dst[t] = T::A_BYTES + b * 1024;
+      dst[t] = kh * T::STEP + T::A_BYTES + b * 1024;
     } else {
-      const int b = q - (T::NIA + T::NIC);
+      int b = q - WK * (T::NIA + T::NIC);
+      const int kh = WK == 1 || WE == W_F16 ? 0 : b / (T::NIS ? T::NIS : 1);
+      b -= kh * T::NIS;
       if constexpr (WE == W_Q4) {                     // (scale, min) word of block b / 2, record b & 1
         const uint32_t r = wrow(p, nB + 64 * (b >> 1) + lane);
         src[t] = ((r >> 6) * p.wG + (p.wk0 >> 5) + (b & 1)) * 1280u + 1024u + (r & 63u) * 4u;
@@ -238,32 +258,48 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
         const uint32_t r = wrow(p, nB + 64 * bb + lane);
         src[t] = ((r >> 6) * p.wG + (p.wk0 >> 6)) * 4224u + 4096u + (r & 62u) * 2u;
       }
-      dst[t] = T::A_BYTES + T::BC_BYTES + b * 256;
+      dst[t] = kh * T::STEP + T::A_BYTES + T::BC_BYTES + b * 256;
     }
   }
   constexpr uint32_t WSTEP = WE == W_F16 ? 128u : (WE == W_Q4 ? 2560u : 4224u);
   const uint32_t smem0 = lds_u32(smem);
-  // issue part `part` (instructions part*NP ..) of step kt into stage st
+  // the step of the stage that this wave's instruction t loads
+  auto half_of = [&](int t) __attribute__((always_inline)) -> uint32_t {
+    if constexpr (WK == 1) return 0u;
+    const int q = NWV * t + wave;
+    if (t < T::WA) return (uint32_t)(q / T::NIA);
+    if (T::WSPLIT ? t < T::WA + T::WC : q < WK * (T::NIA + T::NIC)) return (uint32_t)((q - WK * T::NIA) / T::NIC);
+    return (uint32_t)((q - WK * (T::NIA + T::NIC)) / (T::NIS ? T::NIS : 1));
+  };
+  // issue part `part` (instructions part*NP ..) of stage kt (WK steps; past the last step, that one again) into slot st
   constexpr int NP = (NW + 2) / 3;
-  auto issue = [&](uint32_t kt, int st, int part) __attribute__((always_inline)) {
-    kt = kt < nk ? kt : nk - 1u;
-    // conv3: the step's tap (uniform; Ci % 64 == 0, so a 64-k step stays inside one tap)
-    uint32_t c0 = 0, kt3 = 0, ky = 0, kx = 0;
-    if constexpr (XG == X_CONV) {
-      const uint32_t kg = kt * DBK, tap = kg / p.Ci;
-      c0 = kg - tap * p.Ci;
-      ky = tap / p.ks;
-      kx = tap - ky * p.ks;
-    }
-    if constexpr (XG == X_CONV3) {
-      const uint32_t kg = kt * DBK, tap = kg / p.Ci, r9 = tap % 9u;
-      c0 = kg - tap * p.Ci;
-      kt3 = tap / 9u;
-      ky = r9 / 3u;
-      kx = r9 - 3u * ky;
+  auto issue = [&](uint32_t stage, int st, int part) __attribute__((always_inline)) {
+    uint32_t ktw[WK], c0w[WK], kt3w[WK], kyw[WK], kxw[WK];
+#pragma unroll
+    for (int w = 0; w < WK; w++) {
+      const uint32_t k1 = stage * WK + w, kt = (k1 < nk ? k1 : nk - 1u) + ks0;
+      // the convolutions: the step's tap (uniform; Ci % 64 == 0, so a 64-k step stays inside one tap)
+      uint32_t c0 = 0, kt3 = 0, ky = 0, kx = 0;
+      if constexpr (XG == X_CONV) {
+        const uint32_t kg = kt * DBK, tap = kg / p.Ci;
+        c0 = kg - tap * p.Ci;
+        ky = tap / p.ks;
+        kx = tap - ky * p.ks;
+      }
+      if constexpr (XG == X_CONV3) {
+        const uint32_t kg = kt * DBK, tap = kg / p.Ci, r9 = tap % 9u;
+        c0 = kg - tap * p.Ci;
+        kt3 = tap / 9u;
+        ky = r9 / 3u;
+        kx = r9 - 3u * ky;
+      }
+      ktw[w] = kt; c0w[w] = c0; kt3w[w] = kt3; kyw[w] = ky; kxw[w] = kx;
     }
 #pragma unroll
     for (int t = part * NP; t < (part + 1) * NP && t < NW; t++) {
+      const bool h1 = WK == 2 && half_of(t) != 0;
+      const uint32_t kt = h1 ? ktw[WK - 1] : ktw[0], c0 = h1 ? c0w[WK - 1] : c0w[0], kt3 = h1 ? kt3w[WK - 1] : kt3w[0],
+                     ky = h1 ? kyw[WK - 1] : kyw[0], kx = h1 ? kxw[WK - 1] : kxw[0];
       const uint32_t m0 = __builtin_amdgcn_readfirstlane(smem0 + st * T::STAGE + dst[t]);
       if (XG == X_CONV3 && t < T::WA) {
         const uint32_t it = (cv_it[t] >> (10 * kt3)) & 1023u;
@@ -278,14 +314,15 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
         const size_t pix = (size_t)((uint32_t)iy >> up) * p.Wi + ((uint32_t)ix >> up);
         dma16a(in ? p.X + (pix * p.Ci + c0) * 2 + src[t] * 2 : p.Z, m0);
       } else if (t < T::WA) dma16(p.X + (size_t)kt * 128u, src[t], m0);
-      else if (T::WSPLIT ? t < T::WA + T::WC : NWV * t + wave < T::NIA + T::NIC) dma16(p.W + (size_t)kt * WSTEP, src[t], m0);
+      else if (T::WSPLIT ? t < T::WA + T::WC : NWV * t + wave < WK * (T::NIA + T::NIC)) dma16(p.W + (size_t)kt * WSTEP, src[t], m0);
       else dma4(p.W + (size_t)kt * WSTEP, src[t], m0);
     }
   };
 
   // ---- fragments
-  const int wm = wave / T::WGN, wn = wave % T::WGN, l32 = lane & 31, hh = lane >> 5, sw = (l32 >> 1) & 7;
-  const int rdA = (wm * WTM + l32) * 128;              // byte offset of the lane's first A row in a stage
+  const int wk = wave / (T::WGN * WGM), wm = wave / T::WGN % WGM, wn = wave % T::WGN, l32 = lane & 31, hh = lane >> 5, sw = (l32 >> 1) & 7;
+  const int rdA = (wm * WTM + l32) * 128;              // byte offset of the lane's first A row in a step
+  const int own = wk * T::STEP;                        // and of this wave's step in a stage
   f32x16 acc[BI][BJ];
 #pragma unroll
   for (int i = 0; i < BI; i++)
@@ -301,17 +338,17 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
     for (int j = 0; j < BJ; j++) rodd |= (wrow(p, nB + wn * WTN + 32 * j + l32) & 1u) << j;
   }
   auto rdA_frag = [&](f16x8 *F, int st, int sub) __attribute__((always_inline)) {
-    const uint8_t *sp = smem + st * T::STAGE + rdA + (((4 * hh + sub) ^ sw) & 7) * 16;
+    const uint8_t *sp = smem + st * T::STAGE + own + rdA + (((4 * hh + sub) ^ sw) & 7) * 16;
 #pragma unroll
     for (int i = 0; i < BI; i++) F[i] = *(const f16x8 *)(sp + i * 32 * 128);
   };
   auto rdB_f16 = [&](f16x8 *F, int st, int sub) __attribute__((always_inline)) {
-    const uint8_t *sp = smem + st * T::STAGE + T::A_BYTES + (wn * WTN + l32) * 128 + (((4 * hh + sub) ^ sw) & 7) * 16;
+    const uint8_t *sp = smem + st * T::STAGE + own + T::A_BYTES + (wn * WTN + l32) * 128 + (((4 * hh + sub) ^ sw) & 7) * 16;
 #pragma unroll
     for (int j = 0; j < BJ; j++) F[j] = *(const f16x8 *)(sp + j * 32 * 128);
   };
   auto rdB_codes = [&](int st) __attribute__((always_inline)) {
-    const uint8_t *sb = smem + st * T::STAGE + T::A_BYTES;
+    const uint8_t *sb = smem + st * T::STAGE + own + T::A_BYTES;
 #pragma unroll
     for (int j = 0; j < BJ; j++) {
       const int col = wn * WTN + 32 * j + l32, blk = col >> 6, cb = col & 63;
@@ -357,12 +394,16 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
       }
     }
   };
+  bool met_slow = false;                               // WK = 2: this lane met a word off the fast path
   auto check_q4 = [&](auto chk) __attribute__((always_inline)) {
     if constexpr (WE == W_Q4 && decltype(chk)::value) {
       fmask = 0;
 #pragma unroll
       for (int j = 0; j < BJ; j++) fmask |= (uint32_t)q4n_fast_ok(bs[j]) << j;
       allfast = __all(fmask == (1u << BJ) - 1u);
+    } else if constexpr (WE == W_Q4 && WK == 2) {
+#pragma unroll
+      for (int j = 0; j < BJ; j++) met_slow |= !q4n_fast_ok(bs[j]);
     }
   };
   auto scales_q4 = [&]() __attribute__((always_inline)) {
@@ -386,11 +427,13 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
     constexpr int NMF = BI * BJ, NRD = BI + (WE == W_F16 ? BJ : 0);
     constexpr int NV = WE == W_F16 ? 0 : (WE == W_Q4 ? 18 * BJ : 16 * BJ);
     constexpr int VPM = (NV + NMF - 1) / NMF;
+    // (WK = 2 has few MFMAs per sub-step: its LDS reads go out first, so they land under the decode)
+    if constexpr (WK == 2) __builtin_amdgcn_sched_group_barrier(0x100, NRD, 0);
 #pragma unroll
     for (int q = 0; q < NMF; q++) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       if (VPM) __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
-      if (q < NRD) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (WK == 1 && q < NRD) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
   };
 
@@ -402,11 +445,11 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
   // q4: when every (scale, min) word the tile reads takes the fast decode (ordinary weights), the K loop runs without
   // the per-step check and the fix-up branch of each sub-step, one straight-line block per sub-step
   bool tile_fast = true;
-  if constexpr (WE == W_Q4) {
+  if constexpr (WE == W_Q4 && WK == 1) {
     // thread t reads column t % TBN in groups t / TBN, + NT / TBN, ...; 16 loads in flight per thread
     constexpr uint32_t GS = T::NT / TBN;
-    const uint32_t ng = p.K >> 5, col = tid % TBN, r = wrow(p, nB + col);
-    const uint8_t *wp = p.W + (size_t)((r >> 6) * p.wG + (p.wk0 >> 5) + tid / TBN) * 1280u + 1024u + (r & 63u) * 4u;
+    const uint32_t ng = nk * (DBK / 32), col = tid % TBN, r = wrow(p, nB + col);
+    const uint8_t *wp = p.W + (size_t)((r >> 6) * p.wG + (p.wk0 >> 5) + ks0 * (DBK / 32) + tid / TBN) * 1280u + 1024u + (r & 63u) * 4u;
     bool ok = true;
     uint32_t g = tid / TBN;
     for (; g + 15 * GS < ng; g += 16 * GS, wp += 16 * GS * 1280u) {
@@ -434,7 +477,7 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
     }
     int st = 0, pst = S - 1;
     uint32_t pk = S - 1;
-    for (uint32_t kt = 0; kt < nk; kt++) {
+    for (uint32_t kt = 0; kt < nk / WK; kt++) {
 #pragma unroll
       for (int sub = 0; sub < 3; sub++) {
         f16x8 *An = FA[(sub + 1) & 1], *Bn = FB[(sub + 1) & 1];
@@ -474,10 +517,44 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
       }
       st = sn;
     }
+    if constexpr (WK == 2) {
+      // an odd number of steps: the first half of the waves takes the last one (its first fragments are read)
+      if ((nk & 1u) && wk == 0) {
+#pragma unroll
+        for (int sub = 0; sub < 4; sub++) {
+          mfma(FA[sub & 1], FB[sub & 1]);
+          if (sub < 3) {
+            rdA_frag(FA[(sub + 1) & 1], st, sub + 1);
+            if constexpr (WE == W_F16) {
+              rdB_f16(FB[(sub + 1) & 1], st, sub + 1);
+            } else {
+              decode(FB[(sub + 1) & 1], sub + 1);
+              fix_q4(FB[(sub + 1) & 1], sub + 1, chk);
+            }
+          }
+        }
+      }
+    }
   };
   if (tile_fast) run(std::false_type{});
   else run(std::true_type{});
   wait_vm<0>();
+  if constexpr (WE == W_Q4 && WK == 2) {
+    // short runs of K do not wait for that look at every word before they start (2.5 us): the loop without the check
+    // notes words off the fast path, and a tile that met one is done again with it
+    if (!__syncthreads_and(!met_slow)) {
+#pragma unroll
+      for (int i = 0; i < BI; i++)
+#pragma unroll
+        for (int j = 0; j < BJ; j++) acc[i][j] = (f32x16){};
+#pragma unroll
+      for (int s = 0; s < S - 1; s++)
+#pragma unroll
+        for (int part = 0; part < 3; part++) issue(s, s, part);
+      run(std::true_type{});
+      wait_vm<0>();
+    }
+  }
   wait_lgkm0();
   stage_barrier();
 
@@ -500,11 +577,39 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
 #pragma unroll
             for (int r = 0; r < 16; r++) {
               const int row = br + 8 * (r >> 2) + 4 * hh + (r & 3);
-              sC[row * CLD + bc2 + l32] = acc[i][j][r];
+              if (WK == 1 || wk == 0) sC[row * CLD + bc2 + l32] = acc[i][j][r];
             }
           }
         }
       __syncthreads();
+      if constexpr (WK == 2) {
+        // the second half of the waves adds its sums (the same lanes' places)
+        if (wk == 1) {
+#pragma unroll
+          for (int i = 0; i < BI; i++)
+#pragma unroll
+            for (int j = 0; j < BJ; j++) {
+              const int br = r0 + i * 32, bc2 = c0 + j * 32;
+              if (br >= 0 && br < T::CR && bc2 >= 0 && bc2 < T::CW) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) sC[(br + 8 * (r >> 2) + 4 * hh + (r & 3)) * CLD + bc2 + l32] += acc[i][j][r];
+              }
+            }
+        }
+        __syncthreads();
+      }
+      if constexpr (SPLIT) {
+        // a slice of K: the fp32 sums to the workspace, [slice][row][column], 16 bytes per thread, written through the
+        // L2 (sc0 sc1: nothing is left to flush when the kernel ends)
+        static_assert(TBN == 128 && T::CR == TBM, "one part");
+        const srsrc pr = stream_rsrc((const uint8_t *)p.part);
+        for (int it = tid; it < TBM * 32; it += T::NT) {
+          const uint32_t row = mB + (it >> 5), c = (it & 31) * 4;
+          if (row < p.M)
+            sys_store128(pr, ((slice * p.M + row) * p.ldp + nB + c) * 4u, *(const u32x4 *)(sC + (it >> 5) * CLD + c));
+        }
+        return;
+      }
 #pragma unroll
       for (int q = 0; q < T::CW / 128; q++)
         epilogue<T::NT>(p, sC + q * 128, CLD, T::CR, mB + v * T::CR, nB + h * T::CW + q * 128, tid);
@@ -512,38 +617,56 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM>::OCC), (DT<WE, TB
     }
 }
 
-template <int WE, int XG, int TBM, int TBN, int NWV = 4, int WGM = 2>
+template <int WE, int XG, int TBM, int TBN, int NWV = 4, int WGM = 2, int WK = 1, bool CANSPLIT = false>
 hipError_t launch_dma_one(const Params &p, hipStream_t s) {
   Params q = p;
   q.tilesM = (p.M - p.mbase + TBM - 1) / TBM;
   q.tilesN = (p.N - p.nbase + TBN - 1) / TBN;
-  hipLaunchKernelGGL((k_gemm_dma<WE, XG, TBM, TBN, NWV, WGM>), dim3(q.tilesM * q.tilesN), dim3(64 * NWV), 0, s, q);
+  const dim3 grid(q.tilesM * q.tilesN * (q.slices > 1 ? q.slices : 1u)), block(64 * NWV);
+  if constexpr (CANSPLIT) {
+    if (q.slices > 1) hipLaunchKernelGGL((k_gemm_dma<WE, XG, TBM, TBN, NWV, WGM, WK, true>), grid, block, 0, s, q);
+    else hipLaunchKernelGGL((k_gemm_dma<WE, XG, TBM, TBN, NWV, WGM, WK, false>), grid, block, 0, s, q);
+  } else {
+    if (q.slices > 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_gemm_dma<WE, XG, TBM, TBN, NWV, WGM, WK, false>), grid, block, 0, s, q);
+  }
   return hipGetLastError();
 }
 
+// the wave layout of a tile: dma_waves (8 waves, two per SIMD and one workgroup per CU, or 4 and two workgroups)
 template <int WE, int XG>
-hipError_t launch_dma_we(const Params &p, unsigned bm, unsigned bn, unsigned cus, hipStream_t s) {
-  if (bm == 256 && bn == 256) return launch_dma_one<WE, XG, 256, 256, 8>(p, s);
-  if (bm == 256 && bn == 128) {
-    // 8 waves (2 x 4, 128 x 32 each), one workgroup per CU; q4, whose 4-wave form fits two workgroups per CU, keeps
-    // that when the grid holds more than one tile per CU (the same dma_wgs the planner scored the tile with)
-    if constexpr (WE == W_Q4) {
-      const uint64_t tiles = (uint64_t)((p.M + 255) / 256) * ((p.N - p.nbase + 127) / 128);
-      if (dma_wgs(WE, 256, 128, tiles, cus) > 1) return launch_dma_one<WE, XG, 256, 128, 4>(p, s);
-    }
-    // f16 weights need no decode, so their 8 waves lay out 4 x 2 (64 x 64 each): 4 LDS fragments per 4 MFMAs
-    // instead of 5 with 2 x 4 (128 x 32 each); conv3 13 x 92 x 160: 214 -> 207.5 us
-    if constexpr (WE == W_F16) return launch_dma_one<WE, XG, 256, 128, 8, 4>(p, s);
-    return launch_dma_one<WE, XG, 256, 128, 8>(p, s);
+hipError_t launch_dma_we(const Params &p, unsigned bm, unsigned bn, unsigned wv, hipStream_t s) {
+  // f16 weights need no decode, so 8 waves over 256 rows lay out 4 x 2 (64 x 64 each): 4 LDS fragments per 4 MFMAs
+  // instead of 5 with 2 x 4 (128 x 32 each); conv3 13 x 92 x 160: 214 -> 207.5 us
+  constexpr int GM = WE == W_F16 ? 4 : 2;
+  if (bn == 256) {
+    if (bm == 256) return launch_dma_one<WE, XG, 256, 256, 8>(p, s);
+    if (bm == 128) return launch_dma_one<WE, XG, 128, 256>(p, s);
+    return hipErrorInvalidValue;
   }
-  if (bm == 128 && bn == 256) return launch_dma_one<WE, XG, 128, 256>(p, s);
-  if (bm == 128 && bn == 128) {
-    // q4 with at most one tile per CU: 8 waves (2 x 4, 64 x 32 each, two per SIMD) instead of 4 at one per SIMD
-    if constexpr (WE == W_Q4) {
-      const uint64_t tiles = (uint64_t)((p.M + 127) / 128) * ((p.N - p.nbase + 127) / 128);
-      if (dma_wgs(WE, 128, 128, tiles, cus) == 1) return launch_dma_one<WE, XG, 128, 128, 8>(p, s);
+  if (bn != 128) return hipErrorInvalidValue;
+  if (bm == 256 && wv == 8) return launch_dma_one<WE, XG, 256, 128, 8, GM>(p, s);
+  if (bm == 128 && wv == 8) return launch_dma_one<WE, XG, 128, 128, 8>(p, s);
+  if (bm == 128 && wv == 4) return launch_dma_one<WE, XG, 128, 128>(p, s);
+  if constexpr (WE == W_Q4) {
+    if (bm == 256 && wv == 4) return launch_dma_one<WE, XG, 256, 128, 4>(p, s);
+  }
+  if constexpr (XG != X_CONV3) {
+    // wv == 2: 8 waves as 1 x 4 over the columns x 2 over K, any 32 rows
+    switch (bm) {
+    case 32: return launch_dma_one<WE, XG, 32, 128, 8, 1, 2, true>(p, s);
+    case 64: return launch_dma_one<WE, XG, 64, 128, 8, 1, 2, true>(p, s);
+    case 96: return launch_dma_one<WE, XG, 96, 128, 8, 1, 2, true>(p, s);
+    case 128: return launch_dma_one<WE, XG, 128, 128, 8, 1, 2, true>(p, s);
+    case 160: return launch_dma_one<WE, XG, 160, 128, 8, 1, 2, true>(p, s);
+    case 192: return launch_dma_one<WE, XG, 192, 128, 8, 1, 2, true>(p, s);
     }
-    return launch_dma_one<WE, XG, 128, 128>(p, s);
+    if constexpr (WE != W_F16) {                       // (two stages of two steps within 160 KB)
+      if (bm == 224) return launch_dma_one<WE, XG, 224, 128, 8, 1, 2, true>(p, s);
+    }
+    if constexpr (WE == W_Q4) {
+      if (bm == 256) return launch_dma_one<WE, XG, 256, 128, 8, 1, 2, true>(p, s);
+    }
   }
   return hipErrorInvalidValue;
 }

@@ -4,9 +4,9 @@
 
 namespace p0k {
 
-hipError_t launch_dma_q4(const Params &p, int xg, unsigned bm, unsigned bn, unsigned cus, hipStream_t s);
-hipError_t launch_dma_q8(const Params &p, int xg, unsigned bm, unsigned bn, unsigned cus, hipStream_t s);
-hipError_t launch_dma_f16(const Params &p, int xg, unsigned bm, unsigned bn, unsigned cus, hipStream_t s);
+hipError_t launch_dma_q4(const Params &p, int xg, unsigned bm, unsigned bn, unsigned wv, hipStream_t s);
+hipError_t launch_dma_q8(const Params &p, int xg, unsigned bm, unsigned bn, unsigned wv, hipStream_t s);
+hipError_t launch_dma_f16(const Params &p, int xg, unsigned bm, unsigned bn, unsigned wv, hipStream_t s);
 
 namespace {
 
@@ -56,6 +56,26 @@ __global__ __launch_bounds__(256) void k_xprep(Params p, uint16_t *xp) {
   uint16_t *dst = xp + (size_t)m * p.K;
 #pragma unroll 2
   for (uint32_t kq = threadIdx.x; kq < k8; kq += 256) *(u32x4 *)(dst + 8 * kq) = xload8<XM, 1>(p, m, RowCtx{0, 0, 0}, 8 * kq);
+}
+
+// The end of a call whose K was split: the slices' fp32 sums, added in slice order, and the epilogue. One workgroup per
+// 16 rows x 128 columns; a thread's two 16-byte pieces of up to 4 slices are in flight together.
+constexpr int SE_ROWS = 16;
+__global__ __launch_bounds__(256) void k_split_epi(Params p) {
+  __shared__ __attribute__((aligned(16))) float sC[SE_ROWS * 132];
+  const uint32_t mB = blockIdx.x * SE_ROWS, nB = blockIdx.y * 128;
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const uint32_t r = (threadIdx.x >> 5) + 8 * i, c = (threadIdx.x & 31) * 4, m = mB + r < p.M ? mB + r : p.M - 1u;
+    const float *src = p.part + (size_t)m * p.ldp + nB + c;
+    const size_t step = (size_t)p.M * p.ldp;
+    f32x4 sum = (f32x4){};
+#pragma unroll 4
+    for (uint32_t q = 0; q < p.slices; q++) sum += *(const f32x4 *)(src + q * step);
+    *(f32x4 *)(sC + r * 132 + c) = sum;
+  }
+  __syncthreads();
+  epilogue<256>(p, sC, 132, SE_ROWS, mB, nB, threadIdx.x);
 }
 
 }  // namespace
@@ -145,11 +165,84 @@ void dma_tile(uint32_t M, uint32_t N, int we, int xg, unsigned cus, unsigned *bm
   }
 }
 
-static hipError_t launch_dma_x(const Params &p, int we, int xg, unsigned bm, unsigned bn, unsigned cus, hipStream_t s) {
+// the tallest tile of the 1 x 4 x 2 wave layout: two stages of two steps within 160 KB
+static unsigned dma_tall(int we) { return we == W_Q4 ? 256u : we == W_Q8 ? 224u : 192u; }
+
+bool dma_tile_ok(int we, unsigned bm, unsigned bn, unsigned wv) {
+  if (bn == 256) return bm == 128 || bm == 256;
+  if (bn != 128 || bm % 32 || bm < 32 || bm > 256) return false;
+  return bm % 128 == 0 && wv != 2 ? true : bm <= dma_tall(we);
+}
+
+// The plan of a call: dma_tile's tile; or, for grids that leave it idle or tiles half empty, a tile of the 1 x 4 x 2 wave
+// layout (any 32 rows x 128 columns), with K in slices where its tiles are fewer than the CUs; or, with f16 weights, an
+// 8-wave 128 x 128 tile. All are estimated, in us, in one form,
+//   rounds of workgroups x (steps x (time of a 64-k step, less where the round leaves CUs idle) + fixed) (+ the slices'
+//   exchange),
+// whose constants are fitted to timed calls (q4, q8 and f16: 250-270 shapes each of 17..2048 rows x 1024..28672 columns x
+// K 1024..14336, convolutions: 36, every tile and 1..8 slices; rms 5-7 %; over those shapes the picks are 1-1.7 % above
+// the best and 1.8 times as fast as dma_tile's). Taken where it is 10 % under the estimate of dma_tile's tile, so that
+// the fit's errors do not pick a slower one. us, before -> after: q4 17 x 4096 x 4096 40.6 -> 11.0, 77 x 6144 x 4096
+// 40.3 -> 16.8, 300 x 4096 x 14336 130 -> 48, 300 x 28672 x 4096 117 -> 88, 1000 x 4096 x 4096 55 -> 45; f16 77 x 6144 x
+// 4096 42.9 -> 16.5; 3x3 convolutions 64 x 64 x 512 -> 512 75.6 -> 38.8, 16 x 16 x 512 -> 512 66.8 -> 15.6.
+struct TileCost { unsigned m, n, wgs; double step, fix, idle; };
+struct SliceCost { double step[8], idle, fix, fix_row, split, split_mb; };   // step: of 32, 64 .. 256 rows
+static double rounds_us(uint64_t wgs, uint64_t slots, double steps, double step, double idle, double fix) {
+  const uint64_t rounds = (wgs + slots - 1) / slots, last = wgs - (rounds - 1) * slots;
+  return (double)(rounds - 1) * (steps * step + fix) + steps * step * (idle + (1.0 - idle) * (double)last / (double)slots) + fix;
+}
+
+void dma_plan(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbytes, unsigned cus, DmaPlan *d) {
+  static const TileCost tiles[4][4] = {
+      {{128, 128, 1, 0.699, 5.32, 0.724}, {256, 128, 1, 1.143, 8.37, 0.375}, {256, 256, 1, 2.016, 13.3, 0.245}, {}},
+      {{128, 128, 2, 0.869, 4.96, 0.630}, {256, 128, 1, 1.000, 6.70, 0.530}, {256, 256, 1, 1.855, 14.2, 0.357}, {}},
+      {{128, 128, 1, 0.521, 3.63, 0.539}, {128, 256, 1, 0.734, 8.52, 0.685}, {256, 128, 1, 0.824, 6.25, 0.506}, {256, 256, 1, 1.708, 13.4, 0.547}},
+      {{128, 128, 1, 0.593, 8.59, 0.831}, {128, 128, 2, 1.170, 10.3, 0.673}, {256, 128, 1, 1.079, 11.3, 0.719}, {}}};
+  static const SliceCost slices[4] = {
+      {{0.308, 0.374, 0.443, 0.512, 0.609, 0.743, 0.831, 0.910}, 0.670, 2.70, 0.020, 2.54, 0.359},
+      {{0.278, 0.336, 0.410, 0.503, 0.711, 0.785, 0.851, 0.0}, 0.644, 2.77, 0.027, 2.49, 0.364},
+      {{0.262, 0.326, 0.536, 0.608, 0.697, 0.761, 0.0, 0.0}, 0.689, 1.77, 0.024, 3.13, 0.341},
+      {{0.289, 0.362, 0.616, 0.695, 0.821, 0.918, 0.0, 0.0}, 0.846, 6.27, 0.026, 2.34, 0.428}};   // f16, the 2-D gather
+  d->wv = 0;
+  d->slices = 1;
+  dma_tile(M, N, we, xg, cus, &d->bm, &d->bn);
+  const uint32_t nk = K / DBK;
+  // (K of a few steps is all fixed cost; conv3 keeps one order of K; quantised convolution weights were not timed)
+  if (M == 0 || N == 0 || nk < 8 || xg == X_CONV3 || (xg == X_CONV && we != W_F16)) return;
+  const int ei = xg == X_CONV ? 3 : we == W_Q4 ? 0 : we == W_Q8 ? 1 : 2;
+  const uint64_t tn = (N + 127) / 128, had = (uint64_t)((M + d->bm - 1) / d->bm) * ((N + d->bn - 1) / d->bn);
+  const unsigned wgs = dma_wgs(we, d->bm, d->bn, had, cus);
+  double best = 0.0;
+  for (const TileCost &c : tiles[ei])
+    if (c.m == d->bm && c.n == d->bn && c.wgs == wgs && c.m) best = 0.9 * (2.0 + rounds_us(had, (uint64_t)cus * wgs, nk, c.step, c.idle, c.fix));
+  if (best == 0.0) return;
+  if (we == W_F16) {
+    const TileCost &c = tiles[ei][0];
+    const double us = 2.0 + rounds_us((uint64_t)((M + 127) / 128) * tn, cus, nk, c.step, c.idle, c.fix);
+    if (us < best) { best = us; *d = DmaPlan{128, 128, 8, 1}; }
+  }
+  const SliceCost &c = slices[ei];
+  for (unsigned bm = 32; bm <= dma_tall(we); bm += 32) {
+    const uint64_t tm = (M + bm - 1) / bm;
+    for (unsigned S = 1; S <= 8; S++) {
+      const uint64_t part = S > 1 ? (uint64_t)S * M * dma_ldp(N) * 4u : 0u;
+      if (S > 1 && (nk / S < 4 || tm * tn * S > 2ull * cus || xbytes + part > DMA_SPLIT_BYTES)) break;
+      const double us = 2.0 + rounds_us(tm * tn * S, cus, (double)nk / S, c.step[bm / 32 - 1], c.idle, c.fix + c.fix_row * bm) +
+                        (S > 1 ? c.split + c.split_mb * 1e-6 * (double)part : 0.0);
+      if (us < best) { best = us; *d = DmaPlan{bm, 128, 2, S}; }
+    }
+  }
+}
+
+static hipError_t launch_dma_x(const Params &p, int we, int xg, unsigned bm, unsigned bn, unsigned wv, unsigned cus,
+                               hipStream_t s) {
+  const uint64_t tiles = (uint64_t)((p.M - p.mbase + bm - 1) / bm) * ((p.N - p.nbase + bn - 1) / bn);
+  if (!wv && bn == 128 && bm % 128) wv = 2;
+  if (!wv) wv = dma_wgs(we, bm, bn, tiles, cus) == 1 ? 8 : 4;
   switch (we) {
-  case W_Q4: return launch_dma_q4(p, xg, bm, bn, cus, s);
-  case W_Q8: return launch_dma_q8(p, xg, bm, bn, cus, s);
-  case W_F16: return launch_dma_f16(p, xg, bm, bn, cus, s);
+  case W_Q4: return launch_dma_q4(p, xg, bm, bn, wv, s);
+  case W_Q8: return launch_dma_q8(p, xg, bm, bn, wv, s);
+  case W_F16: return launch_dma_f16(p, xg, bm, bn, wv, s);
   }
   return hipErrorInvalidValue;
 }
@@ -173,19 +266,25 @@ void dma_tail(uint32_t M, uint32_t N, int we, unsigned bm, unsigned bn, unsigned
   dma_tile(M, N - *ncut, we, X_F16, cus, bm2, bn2);
 }
 
-hipError_t launch_gemm_dma(const Params &p, int we, int xg, unsigned bm, unsigned bn, unsigned cus, bool tail,
-                           hipStream_t s) {
+hipError_t launch_gemm_dma(const Params &p, int we, int xg, const DmaPlan &d, unsigned cus, bool tail, hipStream_t s) {
+  const unsigned bm = d.bm, bn = d.bn;
+  if (p.slices > 1) {
+    hipError_t e = launch_dma_x(p, we, xg, bm, bn, 2, cus, s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_split_epi, dim3((p.M + SE_ROWS - 1) / SE_ROWS, p.ldp / 128), dim3(256), 0, s, p);
+    return hipGetLastError();
+  }
   uint32_t ncut = p.N;
   unsigned bm2 = bm, bn2 = bn;
-  if (xg == X_F16 && tail) dma_tail(p.M, p.N, we, bm, bn, cus, &ncut, &bm2, &bn2);
-  if (ncut >= p.N) return launch_dma_x(p, we, xg, bm, bn, cus, s);
+  if (xg == X_F16 && tail && d.wv == 0) dma_tail(p.M, p.N, we, bm, bn, cus, &ncut, &bm2, &bn2);
+  if (ncut >= p.N) return launch_dma_x(p, we, xg, bm, bn, d.wv, cus, s);
   Params a = p, b = p;
   a.N = ncut;                                                 // epilogue bounds: the first launch's columns only
   a.nbase = 0;
   b.nbase = ncut;
-  hipError_t e = launch_dma_x(a, we, xg, bm, bn, cus, s);
+  hipError_t e = launch_dma_x(a, we, xg, bm, bn, 0, cus, s);
   if (e != hipSuccess) return e;
-  return launch_dma_x(b, we, xg, bm2, bn2, cus, s);
+  return launch_dma_x(b, we, xg, bm2, bn2, 0, cus, s);
 }
 
 }  // namespace p0k

@@ -4,11 +4,11 @@
 
 namespace p0k {
 
-hipError_t launch_dma_q4(const Params &p, int xg, unsigned bm, unsigned bn, unsigned cus, hipStream_t s) {
+hipError_t launch_dma_q4(const Params &p, int xg, unsigned bm, unsigned bn, unsigned wv, hipStream_t s) {
   switch (xg) {
-  case X_F16: return launch_dma_we<W_Q4, X_F16>(p, bm, bn, cus, s);
-  case X_CONV: return launch_dma_we<W_Q4, X_CONV>(p, bm, bn, cus, s);
-  case X_CONV3: return launch_dma_we<W_Q4, X_CONV3>(p, bm, bn, cus, s);
+  case X_F16: return launch_dma_we<W_Q4, X_F16>(p, bm, bn, wv, s);
+  case X_CONV: return launch_dma_we<W_Q4, X_CONV>(p, bm, bn, wv, s);
+  case X_CONV3: return launch_dma_we<W_Q4, X_CONV3>(p, bm, bn, wv, s);
   }
   return hipErrorInvalidValue;
 }

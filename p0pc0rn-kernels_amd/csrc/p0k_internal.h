@@ -8,7 +8,8 @@ namespace p0k {
 struct Params;
 enum { K_MFMA = 0, K_GEMV = 1, K_GEMV_MF = 2, K_MFMA_DMA = 3, K_GEMV_SN = 4 };
 // kernel choice of one call: GEMV items are (128-column tile) x (K slice of KS), S slices per tile
-struct Plan { int kernel, we, xm; unsigned bm, bn, S, KS; bool mx, narrow; };
+// (load-to-LDS GEMM: S slices of K, wv waves, 0: by the tile)
+struct Plan { int kernel, we, xm; unsigned bm, bn, S, KS; bool mx, narrow; unsigned wv; };
 // What the kernel choice depends on besides the call: the device's CU count and the P0K_* tuning switches of the
 // environment. A context reads them once (at creation and on p0k_ctx_reload_env); calls without a context read
 // them on the spot.
@@ -21,7 +22,8 @@ struct Tuning {
   bool gemv_narrow = true;     // P0K_GEMV_NARROW=0: no 64-column decode items (a K split fills the GPU instead)
   int gemv_sn = -1;            // P0K_GEMV_SN=0|1: short-call decode items of 16 rows never / wherever they apply
   bool mfma_reg = false;       // P0K_MFMA_KERNEL=reg: the register-staged MFMA kernel
-  unsigned tile_m = 0, tile_n = 0;   // P0K_MFMA_TILE=MxN
+  unsigned tile_m = 0, tile_n = 0, tile_wv = 0;   // P0K_MFMA_TILE=MxN[xWAVES]
+  unsigned split = 0;          // P0K_MFMA_SPLIT=n: slices of K of the load-to-LDS kernel (1: none, 0: not set)
   bool dma_tail = true;        // P0K_DMA_TAIL=0: one launch for a mostly empty last round
   int attn_bq = 0;             // P0K_ATTN_BQ=128|256
   int attn_split = -1;         // P0K_ATTN_SPLIT=0|1: attention over runs of keys never / for every call

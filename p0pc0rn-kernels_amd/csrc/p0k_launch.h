@@ -23,8 +23,14 @@ void dma_tail(uint32_t M, uint32_t N, int we, unsigned bm, unsigned bn, unsigned
 // tile per CU; 4 waves, two per CU, otherwise): the planner scores tiles with it and the launcher picks the wave count
 unsigned dma_wgs(int we, unsigned m, unsigned n, uint64_t tiles, unsigned cus);
 hipError_t launch_xprep(const Params &p, int xm, uint16_t *xp, hipStream_t s);
-// cus: the device's CU count; tail: allow the column split of dma_tail
-hipError_t launch_gemm_dma(const Params &p, int we, int xg, unsigned bm, unsigned bn, unsigned cus, bool tail, hipStream_t s);
+// the plan of a load-to-LDS call: tile, waves (0: as dma_wgs says), slices of K
+struct DmaPlan { unsigned bm, bn, wv, slices; };
+constexpr uint64_t DMA_SPLIT_BYTES = 31ull << 20;   // X' and partial sums of a split call at most (the scratch array's room)
+bool dma_tile_ok(int we, unsigned bm, unsigned bn, unsigned wv);   // a tile of the load-to-LDS kernel
+void dma_plan(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbytes, unsigned cus, DmaPlan *d);
+inline uint32_t dma_ldp(uint32_t N) { return (N + 127u) / 128u * 128u; }   // row length of the partial sums
+// cus: the device's CU count; tail: allow the column split of dma_tail. p.slices > 1: p.part holds slices * M * ldp floats
+hipError_t launch_gemm_dma(const Params &p, int we, int xg, const DmaPlan &d, unsigned cus, bool tail, hipStream_t s);
 // decode GEMV (M <= 16, prologue f16 / rms / lnmod): items of 128 ws columns x K/S; S > 1 needs the workspace
 // (part: S*M*N floats, cnt: one zeroed counter per 128-column tile). mf: the matrix-core variant (2 <= M <= 16);
 // mq4: with q4 weights, its form without X' staging (k_gemv_mq4); mx: q4 at M = 2 takes the stream kernel's

@@ -503,6 +503,27 @@ struct WsSource {
     *out = c->ws_x;
     return P0K_OK;
   }
+  // partial sums of a GEMM over slices of K, beside `xbytes` of X': null where the call has to do without (as xws_if;
+  // the planner keeps both inside the scratch array)
+  int slices_if(uint64_t xbytes, uint64_t need, float **out) {
+    *out = nullptr;
+    if (scratch) {
+      xbytes = (xbytes + 255) / 256 * 256;
+      if (xbytes + need <= SCRATCH_BYTES - SCRATCH_WS) *out = (float *)(scratch + SCRATCH_WS + xbytes);
+      return P0K_OK;
+    }
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(c->stream, &cs), "hipStreamIsCapturing");
+    if (cs != hipStreamCaptureStatusNone) {
+      std::lock_guard<std::mutex> lk(c->mu);
+      if (!c->own_capture || need > c->ws_part_bytes) return P0K_OK;
+    }
+    const int r = grow_ws(c, (void **)&c->ws_part, &c->ws_part_bytes, &c->ws_part_epoch, need, "split");
+    if (r == P0K_OK) *out = c->ws_part;
+    if (r != P0K_E_NOMEM) return r;
+    (void)hipGetLastError();
+    return P0K_OK;
+  }
   // the X' workspace of a call that can do with less than `need`, or without: what there is of it, null where none can
   // be had (a caller captures the stream, nothing to grow during a capture, or no memory)
   int xws_if(uint64_t need, void **out, uint64_t *have) {
@@ -541,7 +562,8 @@ struct WsSource {
 // workspace, and the gather reads plain fp16 pixels (the register-staged kernel applies them once per tap and column
 // tile). A workspace smaller than the image takes it in bands of output rows, each with the input rows that its taps
 // touch (the K order, and so the bits, do not change); without room for one output row, the register-staged kernel.
-static hipError_t conv_gn(const p0k::Params &p0, const p0k::Plan &plan, const p0k::Tuning &tune, WsSource &ws, int *err) {
+static hipError_t conv_gn(const p0k::Params &p0, const p0k::Plan &plan, p0k::DmaPlan d, const p0k::Tuning &tune, WsSource &ws,
+                          int *err) {
   p0k::Params p = p0;
   const uint64_t line = (uint64_t)p.Wi * p.Ci * 2u;                 // bytes of an input row
   const uint32_t rows = (p.M - 1) / p.Wo + 1, up = p.flags & p0k::F_UP2 ? 1u : 0u;
@@ -556,6 +578,11 @@ static hipError_t conv_gn(const p0k::Params &p0, const p0k::Plan &plan, const p0
     unsigned bm, bn;
     p0k::mfma_tile(p.M, p.N, tune.cus, &bm, &bn);
     return p0k::launch_gemm_mfma(p, plan.we, plan.xm, bm, bn, ws.c->stream);
+  }
+  if (band < rows && d.slices > 1) {                                // (partial sums are rows of the whole call)
+    d = p0k::DmaPlan{0, 0, 0, 1};
+    p.slices = 1;
+    p0k::dma_tile(p.M, p.N, plan.we, p0k::X_CONV, tune.cus, &d.bm, &d.bn);
   }
   for (uint64_t y0 = 0; y0 < rows; y0 += band) {
     const uint64_t y1 = std::min<uint64_t>(rows, y0 + band);
@@ -572,7 +599,7 @@ static hipError_t conv_gn(const p0k::Params &p0, const p0k::Plan &plan, const p0
     }
     p.mbase = (uint32_t)(y0 * p.Wo);
     p.M = (uint32_t)std::min<uint64_t>(p0.M, y1 * p.Wo);
-    hipError_t e = p0k::launch_gemm_dma(p, plan.we, P0K_X_CONV, plan.bm, plan.bn, tune.cus, false, ws.c->stream);
+    hipError_t e = p0k::launch_gemm_dma(p, plan.we, P0K_X_CONV, d, tune.cus, false, ws.c->stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -617,6 +644,19 @@ static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
   p.GT = (const uint16_t *)a->gt_buf;
   HIPCHK(hipSetDevice(c->device), "hipSetDevice");
   hipError_t e;
+  p0k::DmaPlan d{plan.bm, plan.bn, plan.wv, plan.S};
+  if (plan.kernel == p0k::K_MFMA_DMA && d.slices > 1) {
+    const uint64_t xbytes = plan.xm == P0K_X_CONV ? (p.flags & p0k::F_GN ? (uint64_t)p.nvox * p.Ci * 2u : 0u)
+                                                  : (plan.xm != P0K_X_F16 ? (uint64_t)a->M * a->K * 2u : 0u);
+    p.ldp = p0k::dma_ldp(a->N);
+    if (int rr = ws.slices_if(xbytes, (uint64_t)d.slices * a->M * p.ldp * sizeof(float), &p.part)) return rr;
+    if (p.part) {
+      p.slices = d.slices;
+    } else {
+      d = p0k::DmaPlan{0, 0, 0, 1};
+      p0k::dma_tile(a->M, a->N, plan.we, plan.xm == P0K_X_CONV ? p0k::X_CONV : p0k::X_F16, tune.cus, &d.bm, &d.bn);
+    }
+  }
   if (plan.kernel == p0k::K_GEMV_SN) {
     e = p0k::launch_gemv_sn(p, plan.we, plan.xm, c->stream);
   } else if (plan.kernel == p0k::K_GEMV || plan.kernel == p0k::K_GEMV_MF) {
@@ -641,14 +681,14 @@ static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
       if (e != hipSuccess) return hip_err(e, "gemm prologue launch");
       p.X = (const uint8_t *)xw;
     }
-    e = p0k::launch_gemm_dma(p, plan.we, P0K_X_CONV3, plan.bm, plan.bn, tune.cus, false, c->stream);
+    e = p0k::launch_gemm_dma(p, plan.we, P0K_X_CONV3, d, tune.cus, false, c->stream);
   } else if (plan.kernel == p0k::K_MFMA_DMA && plan.xm == P0K_X_CONV) {
     p.Z = (const uint8_t *)ws.zero();
     if (p.flags & p0k::F_GN) {
-      e = conv_gn(p, plan, tune, ws, &r);
+      e = conv_gn(p, plan, d, tune, ws, &r);
       if (r) return r;
     } else {
-      e = p0k::launch_gemm_dma(p, plan.we, P0K_X_CONV, plan.bm, plan.bn, tune.cus, false, c->stream);
+      e = p0k::launch_gemm_dma(p, plan.we, P0K_X_CONV, d, tune.cus, false, c->stream);
     }
   } else if (plan.kernel == p0k::K_MFMA_DMA) {
     if (plan.xm != P0K_X_F16) {
@@ -662,7 +702,7 @@ static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
       p.ldx = a->K;
       p.kx0 = 0;
     }
-    e = p0k::launch_gemm_dma(p, plan.we, P0K_X_F16, plan.bm, plan.bn, tune.cus, tune.dma_tail, c->stream);
+    e = p0k::launch_gemm_dma(p, plan.we, P0K_X_F16, d, tune.cus, tune.dma_tail, c->stream);
   } else {
     e = p0k::launch_gemm_mfma(p, plan.we, plan.xm, plan.bm, plan.bn, c->stream);
   }

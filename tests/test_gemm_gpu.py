@@ -279,7 +279,7 @@ def _adversarial_q8(rows, K, seed):
 
 @pytest.mark.parametrize("enc", ["q4g32a.t64", "q8g64s.t64"])
 @pytest.mark.parametrize("path", ["gemv", "gemv_short", "gemv_short4", "gemv_mx2", "gemv_mx8", "gemv_mx16", "gemv_mfma",
-                                  "gemv_mfma_staged", "mfma"])
+                                  "gemv_mfma_staged", "mfma", "mfma_halves", "mfma_slices"])
 def test_dequant_bit_exact(dev, enc, path, monkeypatch):
     """X = unit rows e_k: each output is ONE product 1.0 * W'[n, k], so the fp16 output is the decoded weight itself,
     which must equal the oracle's f16(f32(q*s + mn)) / f16(q*s) bit for bit — on random codes and scale words chosen
@@ -295,12 +295,15 @@ def test_dequant_bit_exact(dev, enc, path, monkeypatch):
         monkeypatch.setenv("P0K_GEMV_MX", "16")
     if path == "gemv_mfma_staged":
         monkeypatch.setenv("P0K_GEMV_MQ4", "0")
+    if path in ("mfma_halves", "mfma_slices"):               # (a tile that meets a slow word is done again)
+        monkeypatch.setenv("P0K_MFMA_TILE", "96x128x2")
+        monkeypatch.setenv("P0K_MFMA_SPLIT", "2" if path == "mfma_slices" else "1")
     rows, K = 128, 256
     wb = _adversarial_q4(rows, K, 3) if enc.startswith("q4") else _adversarial_q8(rows, K, 4)
     want = oracle.dequant(enc, wb, rows, K)                                  # [rows][K] fp16 bits
     dw = dev.upload(wb)
     try:
-        M = {"gemv": 1, "gemv_short": 1, "gemv_short4": 4, "gemv_mx2": 2, "gemv_mx8": 8, "gemv_mx16": 16, "gemv_mfma": 16, "gemv_mfma_staged": 16, "mfma": K}[path]
+        M = {"gemv": 1, "gemv_short": 1, "gemv_short4": 4, "gemv_mx2": 2, "gemv_mx8": 8, "gemv_mx16": 16, "gemv_mfma": 16, "gemv_mfma_staged": 16}.get(path, K)
         got = np.zeros((K, rows), np.uint16)
         for k0 in range(0, K, M):
             X = np.zeros((M, K), np.float32)
@@ -422,15 +425,16 @@ def test_conv2d_gather_every_tile(dev, kw, monkeypatch):
         a, b = c.bufs["pv"][:kw["Ci"]], c.bufs["pv"][kw["Ci"]:]
         tol += np.abs(c.Wt).max() * 2.0 ** -10 * (np.abs(c.X).max() * np.abs(a).max() + np.abs(b).max())
     outs = []
-    for t in MFMA_TILES:
+    for t in MFMA_TILES + ["32x128x2", "96x128x2", "192x128x2/3"]:
         banner(f"conv2d gather tile {t} {kw}")
-        monkeypatch.setenv("P0K_MFMA_TILE", t)
+        monkeypatch.setenv("P0K_MFMA_TILE", t.split("/")[0])
+        monkeypatch.setenv("P0K_MFMA_SPLIT", t.split("/")[1] if "/" in t else "1")
         got = c.run_device(dev)
         assert c.kernel == "mfma_dma"
         err = np.abs(to_float(got) - want)
         assert np.all(err <= tol), f"conv2d gather tile {t} {kw}: max {(err / tol).max()} of the tolerance"
         outs.append(got)
-    for o in outs[1:]:
+    for o in outs[1:len(MFMA_TILES)]:
         assert np.array_equal(o, outs[0])
 
 
@@ -582,6 +586,71 @@ def test_every_mfma_tile_matches_oracle(dev, kw, kernel, monkeypatch):
         outs.append(got)
     for o in outs[1:]:
         assert np.array_equal(o, outs[0])
+
+
+# the 1 x 4 x 2 wave layout (any 32 rows x 128 columns, alternate 64-k steps on the two halves of the waves) and K in
+# slices: tiles of every height with ragged M and N, odd and even numbers of steps (one step: the first half alone),
+# slices of unequal length, every epilogue family
+SLICE_CASES = [
+    dict(enc="q4g32a.t64", epi="f16", M=17, N=130, K=64),
+    dict(enc="q4g32a.t64", epi="swiglu", M=33, N=392, K=576, bias=True),
+    dict(enc="q4g32a.t64", xmode="rms", epi="heads", M=77, N=512, K=640, Hq=2, Hkv=1, Ltot=90, row_off=5),
+    dict(enc="q4g32a.t64", epi="onormgate", M=129, N=256, K=448),
+    dict(enc="q8g64s.t64", xmode="rms", epi="resadd", M=97, N=328, K=704, gate=True),
+    dict(enc="q8g64s.t64", epi="bias", M=250, N=200, K=512, res=True, wk0=64),
+    dict(enc="f16", xmode="lnmod", epi="f32", M=161, N=264, K=832),
+    dict(enc="f16", epi="f16", M=40, N=131, K=192, ld_pad=8),
+]
+
+
+@pytest.mark.parametrize("slices", [1, 3, 8])
+@pytest.mark.parametrize("kw", SLICE_CASES, ids=lambda k: f"{k['enc']}-{k.get('xmode', 'f16')}-{k['epi']}-K{k['K']}")
+def test_k_halves_and_slices_match_oracle(dev, kw, slices, monkeypatch):
+    c = make_case(seed=27, **kw)
+    want = c.run_oracle()
+    monkeypatch.setenv("P0K_MFMA_SPLIT", str(slices))
+    tall = {"q4g32a.t64": 256, "q8g64s.t64": 224, "f16": 192}[kw["enc"]]
+    for bm in range(32, tall + 1, 32):
+        banner(f"tile {bm}x128x2 slices {slices} {kw}")
+        monkeypatch.setenv("P0K_MFMA_TILE", f"{bm}x128x2")
+        t = dev.select_tile(c.args(lambda n: c.bufs[n]))
+        assert (t["kernel"], t["BM"], t["BN"]) == ("mfma_dma", bm, 128)
+        got = c.run_device(dev)
+        assert_close(got, want, fp16=want.dtype == np.uint16, what=f"tile {bm} slices {slices}")
+        assert np.array_equal(c.run_device(dev), got), "a second run differs"
+
+
+def test_slices_planned_noalloc_and_captured(dev):
+    """The planner's own choice for a short prompt (tiles of the K-halves layout, K in slices): eager, allocation-free
+    (the same bits) and replayed from a graph captured by a context with no workspace yet (unsplit there), against the
+    oracle."""
+    c = make_case(enc="q4g32a.t64", xmode="rms", epi="bias", M=77, N=512, K=4096, seed=28, wscale=0.02)
+    banner("slices: planned call")
+    a = c.args(lambda n: c.bufs[n])
+    assert dev.select_tile(a)["BM"] < 128
+    want = c.run_oracle()
+    got = c.run_device(dev)
+    assert_close(got, want, what="planned slices")
+    d = {k: dev.upload(v) for k, v in c.bufs.items()}
+    own = p0k.Device(0)
+    try:
+        dev.gemm_noalloc(c.args(lambda n: d[n]))
+        assert np.array_equal(dev.read(d["y"], np.uint16, got.size), got)
+        e = {k: own.upload(v) for k, v in c.bufs.items()}
+        small = make_case(enc="q4g32a.t64", xmode="rms", epi="bias", M=77, N=64, K=4096, seed=29, wscale=0.02)
+        small.run_device(own)                       # sizes the X' workspace, and a smaller one for the slices
+        own.graph_begin()
+        own.gemm(c.args(lambda n: e[n]))
+        g = own.graph_end()
+        for _ in range(3):
+            own.upload(np.zeros_like(c.bufs["y"]), e["y"])
+            own.graph_launch(g)
+            assert_close(own.read(e["y"], np.uint16, got.size), want, what="captured")
+        own.graph_destroy(g)
+    finally:
+        for b in d.values():
+            dev.free(b)
+        own.close()
 
 
 @pytest.mark.parametrize("kw", [dict(enc="q4g32a.t64", xmode="lnmod", epi="heads", M=4096, N=4352, K=128, Hq=32, Hkv=1),
