@@ -120,6 +120,35 @@ def test_attention_matches_oracle(dev, c, bq, monkeypatch):
             dev.free(d)
 
 
+# Causal grids of more blocks than CUs, longest blocks first: heads a multiple of 8 (an XCD's own) and not, all blocks
+# resident at once (the second on each CU in the opposite order) and more, a valid length that levels the work
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,L,nvalid", [(40, 8, 900, 900), (35, 7, 1000, 990), (48, 6, 1500, 700), (72, 9, 513, 513)])
+def test_attention_causal_block_order(dev, Hq, Hkv, L, nvalid):
+    """Sampled rows of every head and block against float64 numpy, with the file's fp16 tolerance (every block of the
+    grid computes some of them, so a block taken twice and another never would show)."""
+    print(f"causal order Hq={Hq} L={L} nvalid={nvalid}", flush=True)
+    c = dict(Hq=Hq, Hkv=Hkv, Lq=L, Lk=L, mode=1, nvalid=nvalid)
+    q, k, v = setup(c, 23)
+    bufs = [dev.upload(a) for a in (q, k, v)] + [dev.buffer(L * Hq * 256)]
+    try:
+        dev.attention({"q": {"buf": bufs[0]}, "k": {"buf": bufs[1]}, "v": {"buf": bufs[2]}, "o": {"buf": bufs[3]}, "Lq": L,
+                       "Lk": L, "Hq": Hq, "Hkv": Hkv, "mode": 1, "nvalid": nvalid})
+        got = oracle.h2f(dev.read(bufs[3], np.uint16, L * Hq * 128)).reshape(L, Hq, 128)
+    finally:
+        for b in bufs:
+            dev.free(b)
+    Q, K, V = (oracle.h2f(a).astype(np.float64).reshape(n, L, 128) for a, n in ((q, Hq), (k, Hkv), (v, Hkv)))
+    rows = sorted({min(L - 1, 128 * b + o) for b in range((L + 127) // 128) for o in (0, 31, 127)})
+    for h in range(Hq):
+        s = Q[h, rows] @ K[h // (Hq // Hkv)].T / np.sqrt(128.0)
+        s = np.where(np.arange(L)[None, :] <= np.minimum(np.array(rows), nvalid - 1)[:, None], s, -np.inf)
+        p = np.exp(s - s.max(1, keepdims=True))
+        want = (p / p.sum(1, keepdims=True)) @ V[h // (Hq // Hkv)]
+        err = np.abs(got[rows, h] - want)
+        assert np.all(err <= 2 ** -8 * np.abs(want).max() + 2 ** -9 * np.abs(want)), f"head {h}: max err {err.max()}"
+
+
 # The few-queries kernel (32-row blocks of a kv head's packed query heads, runs of 32-key tiles over 4 waves): rows and
 # keys at the edges of its blocks, tiles and 128-key sets, one run and several, every mask mode
 FEW = [dict(Hq=h, Hkv=k, Lq=q, Lk=n, mode=m, nvalid=v, cap=cap) for h, k, q, n, m, v, cap in [
