@@ -58,6 +58,7 @@ Tuning tuning_from_env(unsigned cus) {
   if (const char *ov = getenv("P0K_GEMV_SLICES")) t.gemv_slices = (unsigned)std::max(0, atoi(ov));
   if (const char *ov = getenv("P0K_GEMV_MX")) t.gemv_mx = (unsigned)std::max(0, atoi(ov));
   if (const char *ov = getenv("P0K_GEMV_NARROW")) t.gemv_narrow = atoi(ov) != 0;
+  if (const char *ov = getenv("P0K_GEMV_XPREP")) t.gemv_xprep = atoi(ov) != 0;
   if (const char *ov = getenv("P0K_GEMV_SN")) t.gemv_sn = atoi(ov) != 0;
   if (const char *ov = getenv("P0K_MFMA_KERNEL")) t.mfma_reg = strcmp(ov, "reg") == 0;
   if (const char *ov = getenv("P0K_MFMA_TILE")) {
@@ -102,6 +103,17 @@ static bool sn_rule(int we, uint32_t N, uint32_t K, uint32_t M, unsigned cus) {
   if (we == P0K_ENC_Q8G64S_T64)
     return K <= 8192u && (M == 1 || (M == 2 ? items <= (uint64_t)cus * 2u : items <= cus));
   return M <= 2 && K <= 8192u && items * 2u <= (uint64_t)cus * (M == 1 ? 3u : 2u);
+}
+
+// Where the matrix-core decode of q4 / q8 gets its rms / lnmod rows materialised by a pass of their own (about 3 us with
+// its launch). us, in every item -> by the pass: q8 (whose fp16 rows stream with the weights; the fused form stages X' of
+// the item behind a barrier) N 4096 K 4096 5 / 16 rows 14.3 / 26.0 -> 11.7 / 13.0, N 28672 K 4096 2 / 12 rows 23.9 / 33.1
+// -> 22.4 / 25.0, K 14336 18.6 -> 18.1 (5 rows), N 2048 K 1024 5 / 16 rows 7.1 / 9.4 -> 7.7 / 8.9; q4 N 28672 K 4096 5 rows
+// 24.1 -> 17.4, N 4096 K 4096 5 / 8 / 16 rows 12.2 / 12.8 / 15.0 -> 11.8 / 11.8 / 12.0, N 4096 K 2048 5 / 16 rows 8.1 /
+// 9.7 -> 8.4 / 8.8, N 4096 K 8192 12.6 -> 13.2 (not taken), N 6144 K 14336 21.3 -> 20.3; lnmod gains more.
+static bool xprep_rule(int we, uint32_t N, uint32_t K, uint32_t M) {
+  if (we == P0K_ENC_Q8G64S_T64) return K >= 2048u || (M >= 12u && K >= 1024u);
+  return (uint64_t)N * K >= 50u * 1000u * 1000u || (K <= 4096u && (uint64_t)M * K >= 32768u);
 }
 
 int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *err, const Tuning &tune) {
@@ -348,8 +360,26 @@ int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *e
       }
     }
   }
+  // f16 weights, 5..16 rows, or fewer where K is past the short-call items: the load-to-LDS GEMM's 32-row tile reads them
+  // 1.2 to 2.5 times as fast as the matrix-core decode (fp16 products summed in fp32 in both). us, 16 rows unless stated:
+  // N 4096 / 9216 / 28672 K 4096 13.6 / 45.6 / 61.8 -> 11.4 / 18.8 / 38.0, N 6144 K 14336 68.3 -> 31.5, N 4096 K 14336
+  // 5 / 16 rows 34.3 / 36.8 -> 22.8 / 23.7, N 2048 K 1024 9.0 -> 6.5
+  bool soft = false, xprep = false;
+  if (kernel == K_GEMV_MF && we == P0K_ENC_F16 && (M >= 5 || K > gemv_sn_kmax(we)) && K >= 1024 && tune.gemv_mf < 0 && !tune.gemv_slices &&
+      !tune.mfma_reg && tune.gemv_xprep != 0 && gemm_dma_ok(p, we, xm, wbytes) && (!xf32 || tune.decode_ws)) {
+    kernel = K_MFMA;
+    soft = xf32;
+    narrow = false;
+  }
+  // q4 / q8 on the matrix cores with fp32 rows: every item applies the prologue to its X again (and q8 then stages it
+  // instead of streaming it with the weights); materialised once, the decode reads fp16 rows
+  if (kernel == K_GEMV_MF && xf32 && we != P0K_ENC_F16 && tune.decode_ws && tune.gemv_xprep != 0 &&
+      (tune.gemv_xprep == 1 || xprep_rule(we, N, K, M)) &&
+      (uint64_t)M * K * 2u + (S > 1 ? (uint64_t)S * M * ((N + 127) / 128) * 512u : 0u) <= DMA_SPLIT_BYTES)
+    soft = xprep = true;
   if (out) *out = p;
   if (plan) {
+    plan->xprep = xprep; plan->soft = soft;
     plan->kernel = kernel; plan->we = we; plan->xm = xm; plan->bm = 16; plan->bn = kernel == K_GEMV_SN ? 16 : narrow ? 64 : 128; plan->mx = mx; plan->narrow = narrow;
     // the load-to-LDS kernel where it applies (P0K_MFMA_KERNEL=reg keeps the register-staged one, for tests)
     if (kernel == K_MFMA && gemm_dma_ok(p, we, xm, wbytes) && !tune.mfma_reg) kernel = plan->kernel = K_MFMA_DMA;

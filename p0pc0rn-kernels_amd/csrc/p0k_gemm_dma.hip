@@ -49,13 +49,13 @@ __global__ __launch_bounds__(256) void k_gnprep(Params p, uint16_t *xp) {
 }
 
 // X' of the rms / lnmod prologues, materialised once: Xp[m][k] = xload8 (the fused prologue's exact values); one
-// workgroup per row, 8 k per thread and step
+// workgroup per row (and 2048 columns, with few rows), 8 k per thread and step
 template <int XM>
 __global__ __launch_bounds__(256) void k_xprep(Params p, uint16_t *xp) {
   const uint32_t k8 = p.K / 8, m = blockIdx.x;
   uint16_t *dst = xp + (size_t)m * p.K;
 #pragma unroll 2
-  for (uint32_t kq = threadIdx.x; kq < k8; kq += 256) *(u32x4 *)(dst + 8 * kq) = xload8<XM, 1>(p, m, RowCtx{0, 0, 0}, 8 * kq);
+  for (uint32_t kq = blockIdx.y * 256 + threadIdx.x; kq < k8; kq += 256 * gridDim.y) *(u32x4 *)(dst + 8 * kq) = xload8<XM, 1>(p, m, RowCtx{0, 0, 0}, 8 * kq);
 }
 
 // The end of a call whose K was split: the slices' fp32 sums, added in slice order, and the epilogue. One workgroup per
@@ -113,8 +113,10 @@ hipError_t launch_xprep(const Params &p, int xm, uint16_t *xp, hipStream_t s) {
     return hipGetLastError();
   }
   if (p.M == 0) return hipSuccess;
-  if (xm == X_RMS) hipLaunchKernelGGL(k_xprep<X_RMS>, dim3(p.M), dim3(256), 0, s, p, xp);
-  else if (xm == X_LNMOD) hipLaunchKernelGGL(k_xprep<X_LNMOD>, dim3(p.M), dim3(256), 0, s, p, xp);
+  // (few rows: a workgroup per 2048 columns, one trip to memory)
+  const dim3 grid(p.M, p.M <= 512 ? (p.K + 2047) / 2048 : 1);
+  if (xm == X_RMS) hipLaunchKernelGGL(k_xprep<X_RMS>, grid, dim3(256), 0, s, p, xp);
+  else if (xm == X_LNMOD) hipLaunchKernelGGL(k_xprep<X_LNMOD>, grid, dim3(256), 0, s, p, xp);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }

@@ -9,7 +9,9 @@ struct Params;
 enum { K_MFMA = 0, K_GEMV = 1, K_GEMV_MF = 2, K_MFMA_DMA = 3, K_GEMV_SN = 4 };
 // kernel choice of one call: GEMV items are (128-column tile) x (K slice of KS), S slices per tile
 // (load-to-LDS GEMM: S slices of K, wv waves, 0: by the tile)
-struct Plan { int kernel, we, xm; unsigned bm, bn, S, KS; bool mx, narrow; unsigned wv; };
+// (decode with fp32 rows: xprep, X' is materialised once; soft: a decode call that is planned with a workspace and has
+// another plan without, Tuning::decode_ws)
+struct Plan { int kernel, we, xm; unsigned bm, bn, S, KS; bool mx, narrow; unsigned wv; bool xprep, soft; };
 // What the kernel choice depends on besides the call: the device's CU count and the P0K_* tuning switches of the
 // environment. A context reads them once (at creation and on p0k_ctx_reload_env); calls without a context read
 // them on the spot.
@@ -26,6 +28,8 @@ struct Tuning {
   unsigned split = 0;          // P0K_MFMA_SPLIT=n: slices of K of the load-to-LDS kernel (1: none, 0: not set)
   bool dma_tail = true;        // P0K_DMA_TAIL=0: one launch for a mostly empty last round
   int attn_bq = 0;             // P0K_ATTN_BQ=128|256
+  int gemv_xprep = -1;         // P0K_GEMV_XPREP=0|1: X' of fp32 rows materialised for the matrix-core decode never / always
+  bool decode_ws = true;       // a decode call may be planned with the X' workspace (the runtime plans again without)
   int attn_split = -1;         // P0K_ATTN_SPLIT=0|1: attention over runs of keys never / for every call
 };
 Tuning tuning_from_env(unsigned cus);

@@ -478,13 +478,14 @@ void scratch_release(int device, const void *owner) {
 struct WsSource {
   p0k_ctx *c;
   uint8_t *scratch;   // non-null: the allocation-free path
+  uint64_t xoff = 0;  // and the bytes of X' at its start, beside which the partial sums lie
   int part(uint64_t need, float **out) {
     if (scratch) {
-      if (need > SCRATCH_BYTES - SCRATCH_WS)
+      if (need > SCRATCH_BYTES - SCRATCH_WS - xoff)
         return set_err(P0K_E_ARG, "gemm_noalloc: the split decode needs " + std::to_string(need) +
                                       " bytes of partials, the scratch array holds " +
                                       std::to_string(SCRATCH_BYTES - SCRATCH_WS));
-      *out = (float *)(scratch + SCRATCH_WS);
+      *out = (float *)(scratch + SCRATCH_WS + xoff);
       return P0K_OK;
     }
     if (int r = grow_ws(c, (void **)&c->ws_part, &c->ws_part_bytes, &c->ws_part_epoch, need, "decode")) return r;
@@ -627,6 +628,17 @@ static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
       if (int rr = check_operand(c, o.b, o.s, o.n)) return rr;
   }
   if (a->M == 0 || a->N == 0) return P0K_OK;
+  void *xsoft = nullptr;
+  if (plan.soft) {
+    // a decode call planned with the X' workspace: the plan without, where it cannot be had
+    const uint64_t need = (uint64_t)a->M * a->K * 2u;
+    uint64_t have = 0;
+    if (int rr = ws.xws_if(need, &xsoft, &have)) return rr;
+    if (!xsoft || have < need) {
+      tune.decode_ws = false;
+      if ((r = p0k::prepare_gemm(a, &p, &plan, &err, tune))) return set_err(r, err);
+    }
+  }
   {
     // a call enqueued while the stream is being captured (p0k_graph_begin, or a caller's own capture of
     // p0k_ctx_stream) may put the current workspaces into a graph: from here on they are kept when replaced
@@ -660,6 +672,16 @@ static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
   if (plan.kernel == p0k::K_GEMV_SN) {
     e = p0k::launch_gemv_sn(p, plan.we, plan.xm, c->stream);
   } else if (plan.kernel == p0k::K_GEMV || plan.kernel == p0k::K_GEMV_MF) {
+    if (plan.xprep) {
+      e = p0k::launch_xprep(p, plan.xm, (uint16_t *)xsoft, c->stream);
+      if (e != hipSuccess) return hip_err(e, "gemm prologue launch");
+      p.X = (const uint8_t *)xsoft;
+      p.ldx = a->K;
+      p.kx0 = 0;
+      p.flags |= p0k::F_XALIGN8;
+      plan.xm = P0K_X_F16;
+      ws.xoff = ((uint64_t)a->M * a->K * 2u + 255) / 256 * 256;
+    }
     const uint32_t tiles = (a->N + 127) / 128;
     float *part = nullptr;
     if (plan.S > 1) {

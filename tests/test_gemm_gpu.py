@@ -258,6 +258,53 @@ def test_narrow_matrix_core_decode(dev, enc, epi, M, N, K, mq4, narrow, monkeypa
                  what=f"{enc} {epi} M={M} N={N} K={K}")
 
 
+# fp32 rows on the matrix-core decode: X' by a pass of its own or in every item (q4 and q8, K split or in 64-column items,
+# a column offset and a padded row), and f16 weights with 5..16 rows (or K past the short-call items) on the load-to-LDS
+# GEMM or the decode
+@pytest.mark.parametrize("xprep", ["0", "1", None])
+@pytest.mark.parametrize("kw", [dict(enc="q4g32a.t64", xmode="rms", epi="swiglu", M=5, N=1024, K=4096, bias=True),
+                                dict(enc="q4g32a.t64", xmode="lnmod", epi="resadd", M=16, N=328, K=2048, ld_pad=8, k0=64),
+                                dict(enc="q8g64s.t64", xmode="rms", epi="heads", M=7, N=512, K=2048, Hq=2, Hkv=1, Ltot=9, row_off=1),
+                                dict(enc="q8g64s.t64", xmode="lnmod", epi="bias", M=12, N=200, K=1024, res=True, wk0=64),
+                                dict(enc="f16", xmode="f16", epi="f32", M=5, N=264, K=1024),
+                                dict(enc="f16", xmode="rms", epi="swiglu", M=16, N=256, K=1280),
+                                dict(enc="f16", xmode="lnmod", epi="f16", M=1, N=130, K=9216)],
+                         ids=lambda k: f"{k['enc']}-{k['xmode']}-{k['epi']}-M{k['M']}-K{k['K']}")
+def test_decode_rows_materialised(dev, kw, xprep, monkeypatch):
+    if xprep is not None:
+        monkeypatch.setenv("P0K_GEMV_XPREP", xprep)
+    c = make_case(seed=95, **kw)
+    banner(f"xprep={xprep} {kw}")
+    got = c.run_device(dev)
+    if kw["enc"] == "f16":
+        assert c.kernel == ("mfma_dma" if xprep != "0" else "gemv_mfma")
+    want = c.run_oracle(weights=oracle.CPU_WEIGHTS)
+    assert_close(got, want, fp16=got.dtype == np.uint16, what=f"xprep={xprep} {kw}")
+    d = {k: dev.upload(v) for k, v in c.bufs.items()}
+    own = p0k.Device(0)
+    try:
+        dev.gemm_noalloc(c.args(lambda n: d[n]))
+        out = c.bufs[c.out]
+        assert np.array_equal(dev.read(d[c.out], out.dtype, out.size), got)
+        e = {k: own.upload(v) for k, v in c.bufs.items()}          # a context without workspaces: captured without X'
+        split = False
+        own.graph_begin()
+        try:
+            own.gemm(c.args(lambda n: e[n]))
+        except p0k.P0kError as err:                # the decode in K slices needs its partial sums before a capture
+            assert "decode workspace must grow" in str(err)
+            split = True
+        g = own.graph_end()
+        if not split:
+            own.graph_launch(g)
+            assert_close(own.read(e[c.out], out.dtype, out.size), want, fp16=got.dtype == np.uint16, what="captured")
+        own.graph_destroy(g)
+    finally:
+        for b in d.values():
+            dev.free(b)
+        own.close()
+
+
 # ------------------------------------------------------------------------------------------------ dequantisation
 def _adversarial_q4(rows, K, seed):
     """random codes with (scale, min) words that include far-apart exponents (the decoder's exact-fp32 path)."""
