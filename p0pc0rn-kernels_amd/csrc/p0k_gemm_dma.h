@@ -427,13 +427,14 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
     constexpr int NMF = BI * BJ, NRD = BI + (WE == W_F16 ? BJ : 0);
     constexpr int NV = WE == W_F16 ? 0 : (WE == W_Q4 ? 18 * BJ : 16 * BJ);
     constexpr int VPM = (NV + NMF - 1) / NMF;
-    // (WK = 2 has few MFMAs per sub-step: its LDS reads go out first, so they land under the decode)
-    if constexpr (WK == 2) __builtin_amdgcn_sched_group_barrier(0x100, NRD, 0);
+    // (with few MFMAs per sub-step the LDS reads go out first, so they land under the decode)
+    constexpr bool FIRST = WK == 2 || NMF == 1;
+    if constexpr (FIRST) __builtin_amdgcn_sched_group_barrier(0x100, NRD, 0);
 #pragma unroll
     for (int q = 0; q < NMF; q++) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       if (VPM) __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
-      if (WK == 1 && q < NRD) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (!FIRST && q < NRD) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
   };
 
@@ -648,6 +649,8 @@ hipError_t launch_dma_we(const Params &p, unsigned bm, unsigned bn, unsigned wv,
   if (bm == 256 && wv == 8) return launch_dma_one<WE, XG, 256, 128, 8, GM>(p, s);
   if (bm == 128 && wv == 8) return launch_dma_one<WE, XG, 128, 128, 8>(p, s);
   if (bm == 128 && wv == 4) return launch_dma_one<WE, XG, 128, 128>(p, s);
+  // (conv3 keeps one order of K, so it has no halves: its short tile is 2 x 4 waves of 32 x 32)
+  if (XG == X_CONV3 && WE == W_F16 && bm == 64) return launch_dma_one<WE, X_CONV3, 64, 128, 8>(p, s);
   if constexpr (WE == W_Q4) {
     if (bm == 256 && wv == 4) return launch_dma_one<WE, XG, 256, 128, 4>(p, s);
   }

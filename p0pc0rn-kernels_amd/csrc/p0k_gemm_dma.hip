@@ -170,7 +170,8 @@ void dma_tile(uint32_t M, uint32_t N, int we, int xg, unsigned cus, unsigned *bm
 // the tallest tile of the 1 x 4 x 2 wave layout: two stages of two steps within 160 KB
 static unsigned dma_tall(int we) { return we == W_Q4 ? 256u : we == W_Q8 ? 224u : 192u; }
 
-bool dma_tile_ok(int we, unsigned bm, unsigned bn, unsigned wv) {
+bool dma_tile_ok(int we, int xg, unsigned bm, unsigned bn, unsigned wv) {
+  if (xg == X_CONV3) return wv != 2 && ((bm % 128 == 0 && bm <= 256) || (bm == 64 && bn == 128 && we == W_F16));
   if (bn == 256) return bm == 128 || bm == 256;
   if (bn != 128 || bm % 32 || bm < 32 || bm > 256) return false;
   return bm % 128 == 0 && wv != 2 ? true : bm <= dma_tall(we);
@@ -209,8 +210,24 @@ void dma_plan(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbyte
   d->slices = 1;
   dma_tile(M, N, we, xg, cus, &d->bm, &d->bn);
   const uint32_t nk = K / DBK;
-  // (K of a few steps is all fixed cost; conv3 keeps one order of K; quantised convolution weights were not timed)
-  if (M == 0 || N == 0 || nk < 8 || xg == X_CONV3 || (xg == X_CONV && we != W_F16)) return;
+  // (K of a few steps is all fixed cost; quantised convolution weights were not timed)
+  if (M == 0 || N == 0 || nk < 8 || (xg != X_F16 && we != W_F16)) return;
+  if (xg == X_CONV3) {
+    // one order of K whatever the clip (no halves, no slices): tiles of 64 and 128 rows x 128 with 8 waves for clips of few
+    // tiles, the same estimate (61 shapes, rms 2-5 %, picks within 0.5 % of the best). us, before -> after: 128 -> 128
+    // 32 x 32 51.3 -> 23.8, 3 x 41 x 123 52.5 -> 27.9, 2 x 92 x 160 53.1 -> 40.6; 256 -> 256 2 x 27 x 101 92.9 -> 46.0
+    static const TileCost c3[4] = {{256, 128, 1, 0.956, 8.14, 0.779}, {128, 128, 2, 1.301, 3.22, 0.613},
+                                   {128, 128, 1, 0.631, 4.45, 0.825}, {64, 128, 1, 0.403, 2.70, 0.857}};
+    const unsigned had = dma_wgs(we, d->bm, d->bn, 1, cus);
+    double best = 0.0;
+    for (const TileCost &c : c3) {
+      const bool old = c.m == d->bm && c.n == d->bn && c.wgs == had;
+      const double us = (old ? 0.95 : 1.0) * rounds_us((uint64_t)((M + c.m - 1) / c.m) * ((N + 127) / 128), (uint64_t)cus * c.wgs, nk,
+                                                       c.step, c.idle, c.fix);
+      if (best == 0.0 || us < best) { best = us; *d = DmaPlan{c.m, c.n, c.wgs == 2 ? 4u : 8u, 1}; }
+    }
+    return;
+  }
   const int ei = xg == X_CONV ? 3 : we == W_Q4 ? 0 : we == W_Q8 ? 1 : 2;
   const uint64_t tn = (N + 127) / 128, had = (uint64_t)((M + d->bm - 1) / d->bm) * ((N + d->bn - 1) / d->bn);
   const unsigned wgs = dma_wgs(we, d->bm, d->bn, had, cus);
@@ -239,7 +256,7 @@ void dma_plan(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbyte
 static hipError_t launch_dma_x(const Params &p, int we, int xg, unsigned bm, unsigned bn, unsigned wv, unsigned cus,
                                hipStream_t s) {
   const uint64_t tiles = (uint64_t)((p.M - p.mbase + bm - 1) / bm) * ((p.N - p.nbase + bn - 1) / bn);
-  if (!wv && bn == 128 && bm % 128) wv = 2;
+  if (!wv && bn == 128 && bm % 128) wv = xg == X_CONV3 ? 8 : 2;
   if (!wv) wv = dma_wgs(we, bm, bn, tiles, cus) == 1 ? 8 : 4;
   switch (we) {
   case W_Q4: return launch_dma_q4(p, xg, bm, bn, wv, s);

@@ -26,7 +26,7 @@ hipError_t launch_xprep(const Params &p, int xm, uint16_t *xp, hipStream_t s);
 // the plan of a load-to-LDS call: tile, waves (0: as dma_wgs says), slices of K
 struct DmaPlan { unsigned bm, bn, wv, slices; };
 constexpr uint64_t DMA_SPLIT_BYTES = 31ull << 20;   // X' and partial sums of a split call at most (the scratch array's room)
-bool dma_tile_ok(int we, unsigned bm, unsigned bn, unsigned wv);   // a tile of the load-to-LDS kernel
+bool dma_tile_ok(int we, int xg, unsigned bm, unsigned bn, unsigned wv);   // a tile of the load-to-LDS kernel
 void dma_plan(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbytes, unsigned cus, DmaPlan *d);
 inline uint32_t dma_ldp(uint32_t N) { return (N + 127u) / 128u * 128u; }   // row length of the partial sums
 // cus: the device's CU count; tail: allow the column split of dma_tail. p.slices > 1: p.part holds slices * M * ldp floats

@@ -437,7 +437,7 @@ def test_conv3_gather_every_tile(dev, enc, pn, monkeypatch):
     c = make_conv3_case(T=3, H=10, W=12, C=64, N=256, pn=pn, enc=enc)
     want = c.run_oracle()
     outs = []
-    for t in MFMA_TILES:
+    for t in MFMA_TILES + (["64x128x8", "128x128x8"] if enc == "f16" else []):
         banner(f"conv3 gather tile {t} enc {enc} pn {pn}")
         monkeypatch.setenv("P0K_MFMA_TILE", t)
         assert dev.select_tile(c.args(lambda n: c.bufs[n]))["kernel"] == "mfma_dma"
@@ -446,6 +446,29 @@ def test_conv3_gather_every_tile(dev, enc, pn, monkeypatch):
         outs.append(got)
     for o in outs[1:]:
         assert np.array_equal(o, outs[0])
+
+
+def test_conv3_planned_tiles_bit_identical(dev):
+    """Clips whose frame count changes the planned tile (64, 128 or 256 rows) give the frames the bits of the whole clip."""
+    T, H, W, C, N = 9, 48, 80, 64, 64
+    c = make_conv3_case(T, H, W, C, N)
+    dw, dx, dy = dev.upload(c.bufs["w"]), dev.upload(c.bufs["x"]), dev.buffer(T * H * W * N * 2)
+    tiles, outs = set(), []
+    try:
+        for nf in (T, 5, 1):
+            banner(f"conv3 planned tiles, {nf} frames a call")
+            a = dict(c.spec, w=dict(c.spec["w"], buf=dw), x={"buf": dx}, y={"buf": dy}, M=nf * H * W)
+            t = dev.select_tile(a)
+            tiles.add((t["kernel"], t["BM"]))
+            for t0 in range(0, T, nf):
+                padL = max(0, t0 - 1)
+                _conv3_call(dev, c, dw, dx, padL * H * W * C * 2, dy, t0 * H * W * N * 2, t0, min(nf, T - t0), padL)
+            outs.append(dev.read(dy, np.uint16, T * H * W * N))
+    finally:
+        for b in (dw, dx, dy):
+            dev.free(b)
+    assert tiles == {("mfma_dma", 256), ("mfma_dma", 128), ("mfma_dma", 64)}, tiles
+    assert np.array_equal(outs[1], outs[0]) and np.array_equal(outs[2], outs[0])
 
 
 @pytest.mark.parametrize("kw", [dict(), dict(stride=2), dict(up2=True), dict(gn=True), dict(ks=1, pad=0),
