@@ -613,7 +613,10 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
       }
 #pragma unroll
       for (int q = 0; q < T::CW / 128; q++)
-        epilogue<T::NT>(p, sC + q * 128, CLD, T::CR, mB + v * T::CR, nB + h * T::CW + q * 128, tid);
+        // (residual rows in flight: fewer where accumulators are still live; the 4-wave tiles have no registers for any)
+        if (NWV == 4 || !epilogue_res<T::NT, (T::CR * T::CW == TBM * TBN ? 4 : 2)>(p, sC + q * 128, CLD, T::CR, mB + v * T::CR,
+                                                                                   nB + h * T::CW + q * 128, tid))
+          epilogue<T::NT>(p, sC + q * 128, CLD, T::CR, mB + v * T::CR, nB + h * T::CW + q * 128, tid);
       if (v + 1 < TBM / T::CR || h + 1 < TBN / T::CW) __syncthreads();
     }
 }

@@ -658,6 +658,36 @@ def test_every_mfma_tile_matches_oracle(dev, kw, kernel, monkeypatch):
         assert np.array_equal(o, outs[0])
 
 
+# epilogues that read Y: whole 16-byte groups, a ragged last group beside whole ones, and rows or bases off that alignment
+RESIDUAL_CASES = [
+    dict(enc="q4g32a.t64", xmode="rms", epi="resadd", M=301, N=204, ld_pad=4, K=192, gate=True),
+    dict(enc="q4g32a.t64", xmode="rms", epi="resadd", M=130, N=203, n0=1, K=192, gate=True),
+    dict(enc="q8g64s.t64", xmode="rms", epi="resadd", M=257, N=264, n0=4, K=128, gate=True, store=True, bias=True),
+    dict(enc="q8g64s.t64", xmode="rms", epi="bias", M=301, N=204, ld_pad=4, K=192, res=True),
+    dict(enc="f16", xmode="lnmod", epi="bias", M=257, N=392, n0=8, K=192, res=True),
+    dict(enc="f16", epi="bias", M=129, N=195, n0=5, K=128, res=True),
+]
+
+
+@pytest.mark.parametrize("kw", RESIDUAL_CASES, ids=lambda k: f"{k['enc']}-{k['epi']}-M{k['M']}-N{k['N']}")
+def test_residual_rows_in_flight_bit_identical(dev, kw, monkeypatch):
+    """The 8-wave tiles read the residual of several rows at once, the 4-wave tile row by row: the same bits and the
+    oracle's result, on every alignment of Y and with a ragged last group of columns."""
+    c = make_case(seed=33, **kw)
+    want = c.run_oracle()
+    outs = []
+    for t in ("128x128x4", "128x128x8", "256x128x8", "128x256", "256x256", "96x128x2"):
+        banner(f"tile {t} {kw}")
+        monkeypatch.setenv("P0K_MFMA_TILE", t)
+        assert dev.select_tile(c.args(lambda n: c.bufs[n]))["kernel"] == "mfma_dma"
+        got = c.run_device(dev)
+        assert_close(got, want, fp16=want.dtype == np.uint16, what=f"tile {t}")
+        if not t.endswith("x2"):  # (its halves of K are added at the end)
+            outs.append(got)
+    for o in outs[1:]:
+        assert np.array_equal(o, outs[0])
+
+
 # the 1 x 4 x 2 wave layout (any 32 rows x 128 columns, alternate 64-k steps on the two halves of the waves) and K in
 # slices: tiles of every height with ragged M and N, odd and even numbers of steps (one step: the first half alone),
 # slices of unequal length, every epilogue family
