@@ -177,13 +177,18 @@ __device__ __forceinline__ void tile_order(const Params &p, uint32_t bid, uint32
 
 // XG: X' rows (X_F16: an fp16 matrix), the conv3 gather (X_CONV3: input voxels [vox][Ci], padding taps read Z) or the
 // 2-D convolution's (X_CONV: input pixels [pix][Ci], any square kernel, stride and padding, optionally 2x up-sampled)
+// X_CONV3H: the conv3 gather with Ci an odd multiple of 32: the two 32-k halves of a step each have a tap of their own, and
+// the half step past K reads zeros for both operands
 // SPLIT: a workgroup takes one of p.slices slices of K and leaves fp32 sums (k_split_epi applies the epilogue)
+constexpr int X_CONV3H = 5;
 template <int WE, int XG, int TBM, int TBN, int NWV, int WGM, int WK, bool SPLIT>
 __global__ __launch_bounds__((64 * NWV))
 __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE, TBM, TBN, NWV, WGM, WK>::OCC)))) void k_gemm_dma(Params p) {
   using T = DT<WE, TBM, TBN, NWV, WGM, WK>;
   constexpr int S = T::S, BI = T::BI, BJ = T::BJ, NW = T::NW;
   constexpr int WTM = T::WTM, WTN = T::WTN;
+  constexpr bool HALF = XG == X_CONV3H, C3 = XG == X_CONV3 || HALF;
+  static_assert(!HALF || (WE == W_F16 && WK == 1 && !SPLIT), "half steps: f16 weights, one order of K");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[T::SMEM];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -191,13 +196,13 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
   tile_order(p, SPLIT ? blockIdx.x % (p.tilesM * p.tilesN) : blockIdx.x, mt, nt);
   const uint32_t mB = (XG == X_CONV ? p.mbase : 0u) + mt * TBM, nB = p.nbase + nt * TBN;
   // the slice of K of this workgroup: steps [k0, k0 + nk) (one slice: all of them)
-  const uint32_t nkt = p.K / DBK, slice = blockIdx.x / (p.tilesM * p.tilesN);
+  const uint32_t nkt = (p.K + (HALF ? DBK / 2 : 0)) / DBK, slice = blockIdx.x / (p.tilesM * p.tilesN);
   const uint32_t ks0 = SPLIT ? nkt * slice / p.slices : 0u, nk = SPLIT ? nkt * (slice + 1) / p.slices - ks0 : nkt;
 
   // ---- per-lane DMA sources (step 0) and per-step advances; instruction t of this wave is number 4 t + wave of
   //      the stage's list (NWV t + wave)
   uint32_t src[NW];                                   // byte offsets from X' / the weights (both < 4 GiB)
-  uint32_t cv_it[XG == X_CONV3 ? T::WA : 1], cv_yx[XG != X_F16 ? T::WA : 1];      // conv3 / conv row contexts
+  uint32_t cv_it[C3 ? T::WA : 1], cv_yx[XG != X_F16 ? T::WA : 1];      // conv3 / conv row contexts
   uint32_t dst[NW];                                   // byte offset inside a stage
 #pragma unroll
   for (int t = 0; t < NW; t++) {
@@ -208,7 +213,7 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
       const uint32_t r = 8 * q + lane / 8, c = (lane & 7) ^ ((r >> 1) & 7);
       uint32_t m = mB + r;
       m = m < p.M ? m : p.M - 1u;
-      if constexpr (XG == X_CONV3) {
+      if constexpr (C3) {
         // (oy | ox << 16) and the input frame of each of the three time taps (10 bits each)
         const RowCtx rc = row_ctx<X_CONV3>(p, m);
         uint32_t itp = 0;
@@ -221,7 +226,7 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
         }
         cv_it[t] = itp;
         cv_yx[t] = (uint32_t)rc.b | ((uint32_t)rc.c << 16);
-        src[t] = 8 * c;
+        src[t] = 8 * (HALF ? c & 3u : c);
       } else if constexpr (XG == X_CONV) {
         // the row's first tap, signed 16 bits each
         const RowCtx rc = row_ctx<X_CONV>(p, m);
@@ -261,6 +266,9 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
       dst[t] = kh * T::STEP + T::A_BYTES + T::BC_BYTES + b * 256;
     }
   }
+  // the half of the step that the lane's 16-byte chunk of X' belongs to (the same for all its instructions: NWV is even),
+  // and its chunk of a weight row
+  const bool hi = ((((uint32_t)lane & 7u) ^ ((4u * wave + lane / 16) & 7u)) & 4u) != 0;
   constexpr uint32_t WSTEP = WE == W_F16 ? 128u : (WE == W_Q4 ? 2560u : 4224u);
   const uint32_t smem0 = lds_u32(smem);
   // the step of the stage that this wave's instruction t loads
@@ -286,7 +294,15 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
         ky = tap / p.ks;
         kx = tap - ky * p.ks;
       }
-      if constexpr (XG == X_CONV3) {
+      if constexpr (HALF) {
+        const uint32_t kg = kt * DBK, tap = kg / p.Ci, c = kg - tap * p.Ci;
+        const bool wrap = c + 32u == p.Ci;             // the second half starts the next tap
+        const uint32_t tap1 = wrap ? tap + 1u : tap, r0 = tap % 9u, r1 = tap1 % 9u;
+        c0 = hi ? (wrap ? 0u : c + 32u) : c;
+        kt3 = hi ? tap1 / 9u : tap / 9u;
+        ky = hi ? r1 / 3u : r0 / 3u;
+        kx = hi ? r1 % 3u : r0 % 3u;
+      } else if constexpr (XG == X_CONV3) {
         const uint32_t kg = kt * DBK, tap = kg / p.Ci, r9 = tap % 9u;
         c0 = kg - tap * p.Ci;
         kt3 = tap / 9u;
@@ -301,19 +317,22 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
       const uint32_t kt = h1 ? ktw[WK - 1] : ktw[0], c0 = h1 ? c0w[WK - 1] : c0w[0], kt3 = h1 ? kt3w[WK - 1] : kt3w[0],
                      ky = h1 ? kyw[WK - 1] : kyw[0], kx = h1 ? kxw[WK - 1] : kxw[0];
       const uint32_t m0 = __builtin_amdgcn_readfirstlane(smem0 + st * T::STAGE + dst[t]);
-      if (XG == X_CONV3 && t < T::WA) {
+      // (HALF: the second half of the last step may lie past K)
+      const bool past = HALF && hi && kt * DBK + DBK > p.K;
+      if (C3 && t < T::WA) {
         const uint32_t it = (cv_it[t] >> (10 * kt3)) & 1023u;
         const int iy = (int)(cv_yx[t] & 0xffffu) + (int)ky - 1, ix = (int)(cv_yx[t] >> 16) + (int)kx - 1;
         const bool in = (uint32_t)iy < p.Hi && (uint32_t)ix < p.Wi;
         const size_t vox = ((size_t)it * p.Hi + (uint32_t)iy) * p.Wi + (uint32_t)ix;
-        dma16a(in ? p.X + (vox * p.Ci + c0) * 2 + src[t] * 2 : p.Z, m0);
+        dma16a(in && !past ? p.X + (vox * p.Ci + c0) * 2 + src[t] * 2 : p.Z, m0);
       } else if (XG == X_CONV && t < T::WA) {
         const uint32_t up = p.flags & F_UP2 ? 1u : 0u;
         const int iy = (int)(int16_t)(cv_yx[t] & 0xffffu) + (int)ky, ix = ((int)cv_yx[t] >> 16) + (int)kx;
         const bool in = (uint32_t)iy < (p.Hi << up) && (uint32_t)ix < (p.Wi << up);
         const size_t pix = (size_t)((uint32_t)iy >> up) * p.Wi + ((uint32_t)ix >> up);
         dma16a(in ? p.X + (pix * p.Ci + c0) * 2 + src[t] * 2 : p.Z, m0);
-      } else if (t < T::WA) dma16(p.X + (size_t)kt * 128u, src[t], m0);
+      } else if (HALF && kt * DBK + DBK > p.K) dma16a(past ? p.Z : p.W + (size_t)kt * WSTEP + src[t], m0);
+      else if (t < T::WA) dma16(p.X + (size_t)kt * 128u, src[t], m0);
       else if (T::WSPLIT ? t < T::WA + T::WC : NWV * t + wave < WK * (T::NIA + T::NIC)) dma16(p.W + (size_t)kt * WSTEP, src[t], m0);
       else dma4(p.W + (size_t)kt * WSTEP, src[t], m0);
     }
@@ -337,13 +356,16 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
 #pragma unroll
     for (int j = 0; j < BJ; j++) rodd |= (wrow(p, nB + wn * WTN + 32 * j + l32) & 1u) << j;
   }
+  // the 8 k of a lane in 16-k sub-step `sub` (chunk of the step; hh: the lane's half). HALF keeps the register-staged
+  // kernel's order, the other path of these calls, so both give the same bits
+  auto chunk = [&](int sub) __attribute__((always_inline)) { return HALF ? 2 * sub + hh : 4 * hh + sub; };
   auto rdA_frag = [&](f16x8 *F, int st, int sub) __attribute__((always_inline)) {
-    const uint8_t *sp = smem + st * T::STAGE + own + rdA + (((4 * hh + sub) ^ sw) & 7) * 16;
+    const uint8_t *sp = smem + st * T::STAGE + own + rdA + ((chunk(sub) ^ sw) & 7) * 16;
 #pragma unroll
     for (int i = 0; i < BI; i++) F[i] = *(const f16x8 *)(sp + i * 32 * 128);
   };
   auto rdB_f16 = [&](f16x8 *F, int st, int sub) __attribute__((always_inline)) {
-    const uint8_t *sp = smem + st * T::STAGE + own + T::A_BYTES + (wn * WTN + l32) * 128 + (((4 * hh + sub) ^ sw) & 7) * 16;
+    const uint8_t *sp = smem + st * T::STAGE + own + T::A_BYTES + (wn * WTN + l32) * 128 + ((chunk(sub) ^ sw) & 7) * 16;
 #pragma unroll
     for (int j = 0; j < BJ; j++) F[j] = *(const f16x8 *)(sp + j * 32 * 128);
   };
@@ -653,11 +675,13 @@ hipError_t launch_dma_we(const Params &p, unsigned bm, unsigned bn, unsigned wv,
   if (bm == 128 && wv == 8) return launch_dma_one<WE, XG, 128, 128, 8>(p, s);
   if (bm == 128 && wv == 4) return launch_dma_one<WE, XG, 128, 128>(p, s);
   // (conv3 keeps one order of K, so it has no halves: its short tile is 2 x 4 waves of 32 x 32)
-  if (XG == X_CONV3 && WE == W_F16 && bm == 64) return launch_dma_one<WE, X_CONV3, 64, 128, 8>(p, s);
+  if constexpr (WE == W_F16 && (XG == X_CONV3 || XG == X_CONV3H)) {
+    if (bm == 64) return launch_dma_one<WE, XG, 64, 128, 8>(p, s);
+  }
   if constexpr (WE == W_Q4) {
     if (bm == 256 && wv == 4) return launch_dma_one<WE, XG, 256, 128, 4>(p, s);
   }
-  if constexpr (XG != X_CONV3) {
+  if constexpr (XG != X_CONV3 && XG != X_CONV3H) {
     // wv == 2: 8 waves as 1 x 4 over the columns x 2 over K, any 32 rows
     switch (bm) {
     case 32: return launch_dma_one<WE, XG, 32, 128, 8, 1, 2, true>(p, s);

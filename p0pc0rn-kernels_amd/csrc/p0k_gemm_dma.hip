@@ -88,8 +88,13 @@ bool gemm_dma_ok(const Params &p, int we, int xm, uint64_t wbytes) {
     if (p.Ci % 64 != 0 || yspan > 32767 || xspan > 32767 || p.Hi > 16383 || p.Wi > 16383) return false;
   } else if (xm == X_CONV3) {
     // 64-k steps inside one tap; input frames of the three time taps packed in 10 bits; (oy, ox) in 16
-    if (p.Ci % 64 != 0 || p.stride > 1024 || p.ks > 1024 || p.Ho > 65535 || p.Wo > 65535 || p.nvox == 0xffffffffu)
+    // f16 weights also with Ci 96, 160, ...: a tap per half step. us, register-staged kernel -> this one: 96 -> 128 channels
+    // 3 x 41 x 123 58.2 -> 24.7 (with PixelNorm 102 -> 32.2), 13 x 92 x 160 216 -> 167 (385 -> 187); 160 -> 160
+    // 13 x 92 x 160 515 -> 477 (757 -> 506). Ci 32 was not timed and stays on the register-staged kernel
+    const bool half = we == W_F16 && p.Ci % 64 == 32 && p.Ci > 64;
+    if ((p.Ci % 64 != 0 && !half) || p.stride > 1024 || p.ks > 1024 || p.Ho > 65535 || p.Wo > 65535 || p.nvox == 0xffffffffu)
       return false;
+    if (half) return wbytes < (1ull << 32) && p.K != 0 && p.K % 32 == 0 && (p.flags & F_WALIGN8);
   } else {
     // 32-bit lane offsets from the X' base
     const uint64_t xbytes = xm == X_F16 ? ((uint64_t)p.M * p.ldx + p.kx0 + p.K) * 2 : (uint64_t)p.M * p.K * 2;
@@ -209,7 +214,7 @@ void dma_plan(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbyte
   d->wv = 0;
   d->slices = 1;
   dma_tile(M, N, we, xg, cus, &d->bm, &d->bn);
-  const uint32_t nk = K / DBK;
+  const uint32_t nk = (K + DBK - 1) / DBK;
   // (K of a few steps is all fixed cost; quantised convolution weights were not timed)
   if (M == 0 || N == 0 || nk < 8 || (xg != X_F16 && we != W_F16)) return;
   if (xg == X_CONV3) {

@@ -8,7 +8,8 @@ hipError_t launch_dma_f16(const Params &p, int xg, unsigned bm, unsigned bn, uns
   switch (xg) {
   case X_F16: return launch_dma_we<W_F16, X_F16>(p, bm, bn, wv, s);
   case X_CONV: return launch_dma_we<W_F16, X_CONV>(p, bm, bn, wv, s);
-  case X_CONV3: return launch_dma_we<W_F16, X_CONV3>(p, bm, bn, wv, s);
+  case X_CONV3:
+    return p.Ci % 64 == 0 ? launch_dma_we<W_F16, X_CONV3>(p, bm, bn, wv, s) : launch_dma_we<W_F16, X_CONV3H>(p, bm, bn, wv, s);
   }
   return hipErrorInvalidValue;
 }

@@ -9,10 +9,11 @@ constexpr int GEMV_MAX_M = 16;
 // MFMA GEMM (any M): bm x bn tiles in {128, 256}^2, 512 threads; mfma_tile picks the tile for a shape
 void mfma_tile(uint32_t M, uint32_t N, unsigned cus, unsigned *bm, unsigned *bn);
 hipError_t launch_gemm_mfma(const Params &p, int we, int xm, unsigned bm, unsigned bn, hipStream_t s);
-// MFMA GEMM with load-to-LDS operands (fp16 rows of X' in memory, or the conv3 gather of input voxels; q4 / q8 / f16
+// MFMA GEMM with load-to-LDS operands (fp16 rows of X' in memory, or the gather of a convolution's input; q4 / q8 / f16
 // weights decoded in registers). gemm_dma_ok: the call qualifies (prologue f16 with 16-byte rows, rms / lnmod
-// materialised by launch_xprep into an M x K fp16 buffer, or conv3 with Ci % 64 == 0, its PixelNorm materialised by
-// launch_xprep over the input voxels; K % 64 == 0). dma_tile picks the tile. xg: X_F16 (rows) or X_CONV3.
+// materialised by launch_xprep into an M x K fp16 buffer, or conv / conv3 with Ci % 64 == 0, its GroupNorm or PixelNorm
+// materialised by launch_xprep over the input; K % 64 == 0). dma_tile picks an unsplit tile of the plain layouts,
+// dma_plan (below) starts from it. xg: X_F16 (rows), X_CONV or X_CONV3.
 bool gemm_dma_ok(const Params &p, int we, int xm, uint64_t wbytes);
 void dma_tile(uint32_t M, uint32_t N, int we, int xg, unsigned cus, unsigned *bm, unsigned *bn);
 // the column split launch_gemm_dma makes for a mostly empty last round: columns [0, ncut) with the chosen tile, the

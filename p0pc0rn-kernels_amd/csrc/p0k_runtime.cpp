@@ -698,7 +698,20 @@ static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
       // PixelNorm + SiLU once per input element into the X' workspace; the gather then reads plain fp16 voxels
       const uint64_t need = (uint64_t)p.nvox * p.Ci * 2u;
       void *xw = nullptr;
-      if (int rr = ws.xws(need, &xw)) return rr;
+      if (p.Ci % 64) {
+        // these channels also run without a workspace: the register-staged kernel applies the prologue in its loop (the
+        // same fp16 values in the same order of K: the same bits)
+        uint64_t have = 0;
+        if (int rr = ws.xws_if(need, &xw, &have)) return rr;
+        if (!xw || have < need) {
+          unsigned bm, bn;
+          p0k::mfma_tile(p.M, p.N, tune.cus, &bm, &bn);
+          e = p0k::launch_gemm_mfma(p, plan.we, plan.xm, bm, bn, c->stream);
+          return e == hipSuccess ? P0K_OK : hip_err(e, "gemm launch");
+        }
+      } else if (int rr = ws.xws(need, &xw)) {
+        return rr;
+      }
       e = p0k::launch_xprep(p, plan.xm, (uint16_t *)xw, c->stream);
       if (e != hipSuccess) return hip_err(e, "gemm prologue launch");
       p.X = (const uint8_t *)xw;

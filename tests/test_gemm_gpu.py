@@ -394,7 +394,7 @@ def _conv3_call(dev, c, dw, xbuf, xoff, ybuf, yoff, t0, nf, padL=0, ks=1):
                        "padL": padL, "ks": ks}})
 
 
-@pytest.mark.parametrize("dims", [(5, 6, 6, 32, 128), (7, 5, 9, 64, 64), (4, 6, 10, 128, 128)])
+@pytest.mark.parametrize("dims", [(5, 6, 6, 32, 128), (7, 5, 9, 64, 64), (4, 6, 10, 128, 128), (5, 6, 9, 96, 64)])
 def test_conv3_chunks_and_ring_bit_identical(dev, dims):
     """test/kernels.test.js:123-145: 2-frame chunks and a 3-frame ring give output bit-identical to the whole clip."""
     T, H, W, C, N = dims
@@ -446,6 +446,52 @@ def test_conv3_gather_every_tile(dev, enc, pn, monkeypatch):
         outs.append(got)
     for o in outs[1:]:
         assert np.array_equal(o, outs[0])
+
+
+@pytest.mark.parametrize("C", [96, 160])
+@pytest.mark.parametrize("pn", [False, True])
+def test_conv3_half_step_taps(dev, C, pn, monkeypatch):
+    """Channels that are an odd multiple of 32 (f16 weights): the halves of a 64-k step belong to two taps and the last half
+    step lies past K. Every tile matches the oracle and gives the bits of the register-staged kernel, for K of all 27 taps
+    and for shorter K with and without that last half step."""
+    c = make_conv3_case(T=3, H=10, W=12, C=C, N=130, pn=pn)
+    for K in (27 * C, 27 * C - 32, 27 * C - 160):
+        c.spec["K"] = K
+        banner(f"conv3 half steps C={C} K={K} pn={pn}")
+        monkeypatch.setenv("P0K_MFMA_KERNEL", "reg")
+        monkeypatch.delenv("P0K_MFMA_TILE", raising=False)
+        reg = c.run_device(dev)
+        monkeypatch.delenv("P0K_MFMA_KERNEL")
+        if K == 27 * C:
+            assert_close(reg, c.run_oracle(), what="register-staged")
+        for t in MFMA_TILES + ["64x128x8", "128x128x8"]:
+            monkeypatch.setenv("P0K_MFMA_TILE", t)
+            assert dev.select_tile(c.args(lambda n: c.bufs[n]))["kernel"] == "mfma_dma"
+            assert np.array_equal(c.run_device(dev), reg), t
+
+
+def test_conv3_half_steps_without_workspace(dev):
+    """PixelNorm with 96 channels where its X' does not fit (the scratch array of a noalloc call, a capture by a context
+    with no workspace yet): the same bits as the ordinary call."""
+    c = make_conv3_case(T=11, H=125, W=128, C=96, N=64, pn=True)
+    assert 11 * 125 * 128 * 96 * 2 > p0k.lib().p0k_gemm_noalloc_scratch_bytes()
+    banner("conv3 half steps without workspace")
+    want = c.run_device(dev)
+    own = p0k.Device(0)
+    try:
+        d = {k: own.upload(v) for k, v in c.bufs.items()}
+        own.gemm_noalloc(c.args(lambda n: d[n]))
+        assert np.array_equal(own.read(d["y"], np.uint16, want.size), want)
+        own.graph_begin()
+        own.gemm(c.args(lambda n: d[n]))
+        g = own.graph_end()
+        for _ in range(3):
+            own.upload(np.zeros_like(c.bufs["y"]), d["y"])
+            own.graph_launch(g)
+            assert np.array_equal(own.read(d["y"], np.uint16, want.size), want), "captured"
+        own.graph_destroy(g)
+    finally:
+        own.close()
 
 
 def test_conv3_planned_tiles_bit_identical(dev):
