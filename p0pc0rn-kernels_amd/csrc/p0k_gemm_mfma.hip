@@ -1,5 +1,5 @@
 // p0k_gemm_mfma.hip — the prefill / convolution path of `gemm` (src/ops/gemm.js:29-257) on gfx950 matrix cores, for the
-// calls that the load-to-LDS kernel does not take (K or Ci no multiple of 64, unaligned rows, no workspace).
+// calls that the load-to-LDS kernel does not take (K or Ci no multiple of 64 but for some conv3, unaligned rows, no workspace).
 //
 // One workgroup (256 threads = 4 waves of 64) computes a TBM x TBN output tile, TBM, TBN in {128, 256}; the waves
 // form a 2 x 2 grid, each owning a (TBM/2) x (TBN/2) block of 32x32 v_mfma_f32_32x32x16_f16 tiles (fp16 in, fp32

@@ -477,11 +477,12 @@ def test_conv3_half_steps_without_workspace(dev):
     assert 11 * 125 * 128 * 96 * 2 > p0k.lib().p0k_gemm_noalloc_scratch_bytes()
     banner("conv3 half steps without workspace")
     want = c.run_device(dev)
+    n = {k: dev.upload(v) for k, v in c.bufs.items()}
     own = p0k.Device(0)
     try:
+        dev.gemm_noalloc(c.args(lambda k: n[k]))
+        assert np.array_equal(dev.read(n["y"], np.uint16, want.size), want)
         d = {k: own.upload(v) for k, v in c.bufs.items()}
-        own.gemm_noalloc(c.args(lambda n: d[n]))
-        assert np.array_equal(own.read(d["y"], np.uint16, want.size), want)
         own.graph_begin()
         own.gemm(c.args(lambda n: d[n]))
         g = own.graph_end()
@@ -491,6 +492,8 @@ def test_conv3_half_steps_without_workspace(dev):
             assert np.array_equal(own.read(d["y"], np.uint16, want.size), want), "captured"
         own.graph_destroy(g)
     finally:
+        for b in n.values():
+            dev.free(b)
         own.close()
 
 
