@@ -172,7 +172,7 @@ typedef struct p0k_device_info {
 int p0k_abi_version(void);
 const char *p0k_last_error(void);            /* message of the last failed call on this thread */
 
-/* ---- context (createGpu) */
+/* ---- context (createGpu). Threads may share one: its calls are enqueued whole, one after the other. */
 int p0k_ctx_create(int device, p0k_ctx **out);
 void p0k_ctx_destroy(p0k_ctx *ctx);
 int p0k_device_info_get(p0k_ctx *ctx, p0k_device_info *out);

@@ -45,6 +45,10 @@ struct p0k_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::mutex mu;
+  // held from the moment a call takes a workspace until its last launch is enqueued (before mu where both are): a call
+  // of several launches hands its X' or partial sums from one to the next, so another thread's launches (or its growing
+  // of the workspace) must not come between them
+  std::mutex enq;
   // pool accounting, as src/core/gpu.js:33-34, 87-138: every live byte is counted; a freed buffer is kept for the next
   // request of exactly the same (16-byte rounded) size while pooled + live stays within the high-water mark + the
   // largest buffer; reused buffers are cleared before they are handed out again.
@@ -628,6 +632,7 @@ static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
       if (int rr = check_operand(c, o.b, o.s, o.n)) return rr;
   }
   if (a->M == 0 || a->N == 0) return P0K_OK;
+  std::lock_guard<std::mutex> order(c->enq);
   void *xsoft = nullptr;
   if (plan.soft) {
     // a decode call planned with the X' workspace: the plan without, where it cannot be had
@@ -923,6 +928,7 @@ int p0k_graph_end(p0k_ctx *c, p0k_graph **out) {
 }
 int p0k_graph_launch(p0k_ctx *c, p0k_graph *g) {
   if (!c || !g) return set_err(P0K_E_ARG, "graph_launch: NULL argument");
+  std::lock_guard<std::mutex> order(c->enq);     // its calls may use the context's workspaces
   HIPCHK(hipGraphLaunch(g->exec, c->stream), "hipGraphLaunch");
   return P0K_OK;
 }
