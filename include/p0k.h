@@ -249,7 +249,11 @@ int p0k_pack_f16(const float *W, uint64_t n, uint16_t *out);
 
 /* ---- HIP graphs: capture the context's stream (e.g. a decode step's gemm calls), then replay it with one launch.
  *      (The reference batches dispatches into command buffers, src/core/gpu.js:203-257; a graph is the HIP form.)
- *      Between begin and end only enqueueing calls may be made (p0k_gemm, p0k_rowstats, p0k_copy). */
+ *      Between begin and end only enqueueing calls may be made (p0k_gemm, p0k_rowstats, p0k_copy).
+ *      A graph may be launched through any context. Its calls may use the workspaces of the context that captured it: a
+ *      launch through another one is then ordered with that context's work (it waits for what that context has enqueued,
+ *      and what that context enqueues afterwards waits for it), and refused with P0K_E_ARG while either stream is being
+ *      captured or once the capturing context is destroyed. */
 typedef struct p0k_graph p0k_graph;
 int p0k_graph_begin(p0k_ctx *ctx);
 int p0k_graph_end(p0k_ctx *ctx, p0k_graph **out);

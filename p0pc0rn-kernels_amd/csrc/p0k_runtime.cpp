@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -41,8 +42,15 @@ void scratch_release(int device, const void *owner);
 
 }  // namespace
 
+// Where a graph finds the context that captured it: ctx is null once that context is destroyed.
+struct p0k_home {
+  std::mutex mu;
+  p0k_ctx *ctx;
+};
+
 struct p0k_ctx {
   int device = 0;
+  std::shared_ptr<p0k_home> home;
   hipStream_t stream = nullptr;
   std::mutex mu;
   // held from the moment a call takes a workspace until its last launch is enqueued (before mu where both are): a call
@@ -72,6 +80,8 @@ struct p0k_ctx {
   // p0k_graph_begin is capturing the stream (its graphs replay in order with the context's work, so calls in them may
   // use workspaces; a capture begun by the caller may replay anywhere)
   bool own_capture = false;
+  // a call of the current p0k_graph_begin .. p0k_graph_end took a workspace: the graph's replays need the stream's order
+  bool capture_ws = false;
   // 256 zero bytes: the padding taps of the load-to-LDS conv3 gather read them
   void *ws_zero = nullptr;
   // workspaces replaced by larger ones while a graph captured after their allocation may still address them: freed
@@ -106,6 +116,8 @@ int p0k_ctx_create(int device, p0k_ctx **out) {
     return set_err(P0K_E_UNSUPPORTED, std::string("ctx_create: this library is built for gfx950, the device is ") + prop.gcnArchName);
   p0k_ctx *c = new p0k_ctx();
   c->device = device;
+  c->home = std::make_shared<p0k_home>();
+  c->home->ctx = c;
   c->tune = p0k::tuning_from_env((unsigned)prop.multiProcessorCount);
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e != hipSuccess) { delete c; return hip_err(e, "hipStreamCreate"); }
@@ -136,6 +148,10 @@ int p0k_ctx_create(int device, p0k_ctx **out) {
 
 void p0k_ctx_destroy(p0k_ctx *c) {
   if (!c) return;
+  {
+    std::lock_guard<std::mutex> lk(c->home->mu);   // (no graph is being launched through another context)
+    c->home->ctx = nullptr;
+  }
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   if (c->owns_scratch) scratch_release(c->device, c);
@@ -484,6 +500,7 @@ struct WsSource {
   uint8_t *scratch;   // non-null: the allocation-free path
   uint64_t xoff = 0;  // and the bytes of X' at its start, beside which the partial sums lie
   int part(uint64_t need, float **out) {
+    c->capture_ws = true;
     if (scratch) {
       if (need > SCRATCH_BYTES - SCRATCH_WS - xoff)
         return set_err(P0K_E_ARG, "gemm_noalloc: the split decode needs " + std::to_string(need) +
@@ -497,6 +514,7 @@ struct WsSource {
     return P0K_OK;
   }
   int xws(uint64_t need, void **out) {
+    c->capture_ws = true;
     if (scratch) {
       if (need > SCRATCH_BYTES - SCRATCH_WS)
         return set_err(P0K_E_ARG, "gemm_noalloc: the prologue needs " + std::to_string(need) +
@@ -512,6 +530,7 @@ struct WsSource {
   // the planner keeps both inside the scratch array)
   int slices_if(uint64_t xbytes, uint64_t need, float **out) {
     *out = nullptr;
+    c->capture_ws = true;
     if (scratch) {
       xbytes = (xbytes + 255) / 256 * 256;
       if (xbytes + need <= SCRATCH_BYTES - SCRATCH_WS) *out = (float *)(scratch + SCRATCH_WS + xbytes);
@@ -534,6 +553,7 @@ struct WsSource {
   int xws_if(uint64_t need, void **out, uint64_t *have) {
     *out = nullptr;
     *have = 0;
+    c->capture_ws = true;
     if (scratch) {
       *out = scratch + SCRATCH_WS;
       *have = std::min<uint64_t>(need, SCRATCH_BYTES - SCRATCH_WS);
@@ -853,9 +873,11 @@ int p0k_attention(p0k_ctx *c, const p0k_attn_args *a) {
     std::lock_guard<std::mutex> lk(c->mu);
     tune = c->tune;
   }
+  std::lock_guard<std::mutex> order(c->enq);
   bool ws = true;
   if (int rr = ws_allowed(c, &ws)) return rr;
   const unsigned runs = tune.attn_bq ? 0u : p0k::attention_runs(p, (int)tune.cus, ws, tune.attn_split);
+  if (runs > 1) c->capture_ws = true;
   hipError_t e = p0k::launch_attention(p, (int)tune.cus, tune.attn_bq, runs, c->ws_attn, c->ws_attn_cnt, c->stream);
   if (e != hipSuccess) return hip_err(e, "attention launch");
   return P0K_OK;
@@ -896,24 +918,36 @@ int p0k_gn_finalize(p0k_ctx *c, const p0k_gn_args *a) { return gn_run(c, a, 2, n
 int p0k_groupnorm_stats(p0k_ctx *c, const p0k_gn_args *a) { return gn_run(c, a, 3, nullptr); }
 
 // ------------------------------------------------------------------------------------------------ graphs
-struct p0k_graph { hipGraph_t graph; hipGraphExec_t exec; };
+// home: the context that captured it; ws: its calls use that context's workspaces; in / out: the events of launches
+// through other contexts
+struct p0k_graph {
+  hipGraph_t graph;
+  hipGraphExec_t exec;
+  std::shared_ptr<p0k_home> home;
+  bool ws;
+  hipEvent_t in = nullptr, out = nullptr;
+};
 
 int p0k_graph_begin(p0k_ctx *c) {
   if (!c) return set_err(P0K_E_ARG, "graph_begin: NULL context");
   HIPCHK(hipSetDevice(c->device), "hipSetDevice");
   HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-  std::lock_guard<std::mutex> lk(c->mu);
+  std::scoped_lock lk(c->enq, c->mu);
   c->own_capture = true;
+  c->capture_ws = false;
   return P0K_OK;
 }
 int p0k_graph_end(p0k_ctx *c, p0k_graph **out) {
   if (!c || !out) return set_err(P0K_E_ARG, "graph_end: NULL argument");
   *out = nullptr;
   hipGraph_t g = nullptr;
-  hipError_t ce = hipStreamEndCapture(c->stream, &g);
+  bool ws;
+  hipError_t ce;
   {
-    std::lock_guard<std::mutex> lk(c->mu);
+    std::scoped_lock lk(c->enq, c->mu);
+    ce = hipStreamEndCapture(c->stream, &g);
     c->own_capture = false;
+    ws = c->capture_ws;
   }
   HIPCHK(ce, "hipStreamEndCapture");
   {
@@ -923,17 +957,48 @@ int p0k_graph_end(p0k_ctx *c, p0k_graph **out) {
   hipGraphExec_t ex = nullptr;
   hipError_t e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
   if (e != hipSuccess) { (void)hipGraphDestroy(g); return hip_err(e, "hipGraphInstantiate"); }
-  *out = new p0k_graph{g, ex};
+  *out = new p0k_graph{g, ex, c->home, ws};
   return P0K_OK;
 }
 int p0k_graph_launch(p0k_ctx *c, p0k_graph *g) {
   if (!c || !g) return set_err(P0K_E_ARG, "graph_launch: NULL argument");
-  std::lock_guard<std::mutex> order(c->enq);     // its calls may use the context's workspaces
+  if (g->ws) {
+    // its calls use the workspaces of the context that captured it: through another context the replay waits for that
+    // context's work so far, and that context's later work for the replay
+    std::lock_guard<std::mutex> lk(g->home->mu);
+    p0k_ctx *o = g->home->ctx;
+    if (!o) return set_err(P0K_E_ARG, "graph_launch: the graph uses workspaces of the context that captured it, which is destroyed");
+    if (o != c) {
+      std::lock_guard<std::mutex> order(o->enq);
+      for (p0k_ctx *q : {o, c}) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        HIPCHK(hipStreamIsCapturing(q->stream, &cs), "hipStreamIsCapturing");
+        if (cs != hipStreamCaptureStatusNone)
+          return set_err(P0K_E_ARG, "graph_launch: a graph that uses workspaces of another context cannot be launched while "
+                                    "either context's stream is captured");
+      }
+      if (!g->in) {
+        HIPCHK(hipSetDevice(o->device), "hipSetDevice");
+        HIPCHK(hipEventCreateWithFlags(&g->in, hipEventDisableTiming), "hipEventCreate");
+      }
+      HIPCHK(hipSetDevice(c->device), "hipSetDevice");
+      if (!g->out) HIPCHK(hipEventCreateWithFlags(&g->out, hipEventDisableTiming), "hipEventCreate");
+      HIPCHK(hipEventRecord(g->in, o->stream), "hipEventRecord");
+      HIPCHK(hipStreamWaitEvent(c->stream, g->in, 0), "hipStreamWaitEvent");
+      HIPCHK(hipGraphLaunch(g->exec, c->stream), "hipGraphLaunch");
+      HIPCHK(hipEventRecord(g->out, c->stream), "hipEventRecord");
+      HIPCHK(hipStreamWaitEvent(o->stream, g->out, 0), "hipStreamWaitEvent");
+      return P0K_OK;
+    }
+  }
+  std::lock_guard<std::mutex> order(c->enq);     // (not between the launches of another thread's call)
   HIPCHK(hipGraphLaunch(g->exec, c->stream), "hipGraphLaunch");
   return P0K_OK;
 }
 void p0k_graph_destroy(p0k_graph *g) {
   if (!g) return;
+  if (g->in) (void)hipEventDestroy(g->in);
+  if (g->out) (void)hipEventDestroy(g->out);
   (void)hipGraphExecDestroy(g->exec);
   (void)hipGraphDestroy(g->graph);
   delete g;

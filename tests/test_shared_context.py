@@ -51,3 +51,59 @@ def test_threads_share_a_context():
     finally:
         dev.close()
         alone.close()
+
+
+@pytest.mark.parametrize("what", ["attention over runs of keys", "X' and slices of K"])
+def test_graph_launched_through_another_context(what):
+    """A graph whose calls use workspaces, replayed through a second context while the first one's own calls use the same
+    workspaces: both keep the bits they have alone, again and again, and the second context refuses the graph once the
+    first is gone."""
+    own, other = p0k.Device(0), p0k.Device(0)
+    print(f"[p0k-test] graph through another context: {what}", flush=True)
+    try:
+        if what.startswith("attention"):
+            Hq, Hkv, Lk = 32, 8, 3777
+            rng = np.random.default_rng(5)
+            calls, outs, size = [], [], Hq * 128
+            for _ in range(2):
+                q, k, v = (own.upload((rng.standard_normal(n * 128)).astype(np.float16)) for n in (Hq, Hkv * Lk, Hkv * Lk))
+                o = own.buffer(size * 2)
+                a = {"q": {"buf": q}, "k": {"buf": k}, "v": {"buf": v}, "o": {"buf": o}, "Lq": 1, "Lk": Lk, "Hq": Hq,
+                     "Hkv": Hkv, "mode": 2, "nvalid": Lk}
+                calls.append(lambda a=a: own.attention(a))
+                outs.append(o)
+        else:
+            cs = [make_case(enc="q4g32a.t64", xmode="rms", epi="f16", M=77, N=512, K=4096, wscale=0.02, seed=s) for s in (45, 46)]
+            ds = [{k: own.upload(v) for k, v in c.bufs.items()} for c in cs]
+            calls = [lambda c=c, d=d: own.gemm(c.args(lambda n: d[n])) for c, d in zip(cs, ds)]
+            outs, size = [d["y"] for d in ds], cs[0].bufs["y"].size
+        want = []
+        for call, o in zip(calls, outs):
+            call()
+            want.append(own.read(o, np.uint16, size))
+        own.graph_begin()
+        calls[0]()
+        g = own.graph_end()
+        zero = np.zeros(size, np.uint16)
+        for rep in range(10):
+            for o in outs:
+                own.upload(zero, o)
+            for _ in range(4):
+                calls[1]()
+                other.graph_launch(g)
+            calls[1]()
+            for o, w in zip(outs, want):                 # (the read waits for the other context's replays too)
+                assert np.array_equal(own.read(o, np.uint16, size), w), f"repetition {rep}"
+        own.graph_launch(g)
+        assert np.array_equal(own.read(outs[0], np.uint16, size), want[0])
+        own.graph_begin()
+        with pytest.raises(p0k.P0kError, match="is captured"):
+            other.graph_launch(g)
+        own.graph_destroy(own.graph_end())
+        own.close()
+        with pytest.raises(p0k.P0kError, match="destroyed"):
+            other.graph_launch(g)
+        p0k.Device.graph_destroy(g)
+    finally:
+        own.close()
+        other.close()
