@@ -77,9 +77,10 @@ struct p0k_ctx {
   // partial rows and counters of attention over runs of keys: a fixed size, allocated with the context
   float *ws_attn = nullptr;
   uint32_t *ws_attn_cnt = nullptr;
-  // p0k_graph_begin is capturing the stream (its graphs replay in order with the context's work, so calls in them may
-  // use workspaces; a capture begun by the caller may replay anywhere)
-  bool own_capture = false;
+  // the id of the capture that p0k_graph_begin began, 0: none (its graphs replay in order with the context's work, so
+  // calls in them may use workspaces; a capture begun by the caller may replay anywhere). An id and not a flag: the
+  // caller may end that capture with the HIP API and begin one of its own
+  unsigned long long own_capture = 0;
   // a call of the current p0k_graph_begin .. p0k_graph_end took a workspace: the graph's replays need the stream's order
   bool capture_ws = false;
   // 256 zero bytes: the padding taps of the load-to-LDS conv3 gather read them
@@ -431,13 +432,15 @@ static int grow_ws(p0k_ctx *c, void **buf, uint64_t *bytes, uint64_t *epoch, uin
   return P0K_OK;
 }
 
-// Whether a call that could do without may use the context's workspaces: not while a caller captures the stream, whose
-// graph may replay on any stream beside the context's own work.
-static int ws_allowed(p0k_ctx *c, bool *ok) {
+// Whether the stream is being captured, and whether a call that could do without may use the context's workspaces: not
+// while a caller captures the stream, whose graph may replay on any stream beside the context's own work.
+static int ws_allowed(p0k_ctx *c, bool *capturing, bool *ok) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  HIPCHK(hipStreamIsCapturing(c->stream, &cs), "hipStreamIsCapturing");
+  unsigned long long id = 0;
+  HIPCHK(hipStreamGetCaptureInfo(c->stream, &cs, &id), "hipStreamGetCaptureInfo");
   std::lock_guard<std::mutex> lk(c->mu);
-  *ok = cs == hipStreamCaptureStatusNone || c->own_capture;
+  *capturing = cs != hipStreamCaptureStatusNone;
+  *ok = !*capturing || (id != 0 && id == c->own_capture);
   return P0K_OK;
 }
 
@@ -536,12 +539,9 @@ struct WsSource {
       if (xbytes + need <= SCRATCH_BYTES - SCRATCH_WS) *out = (float *)(scratch + SCRATCH_WS + xbytes);
       return P0K_OK;
     }
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    HIPCHK(hipStreamIsCapturing(c->stream, &cs), "hipStreamIsCapturing");
-    if (cs != hipStreamCaptureStatusNone) {
-      std::lock_guard<std::mutex> lk(c->mu);
-      if (!c->own_capture || need > c->ws_part_bytes) return P0K_OK;
-    }
+    bool capturing, ok;
+    if (int rr = ws_allowed(c, &capturing, &ok)) return rr;
+    if (!ok || (capturing && need > c->ws_part_bytes)) return P0K_OK;
     const int r = grow_ws(c, (void **)&c->ws_part, &c->ws_part_bytes, &c->ws_part_epoch, need, "split");
     if (r == P0K_OK) *out = c->ws_part;
     if (r != P0K_E_NOMEM) return r;
@@ -559,16 +559,13 @@ struct WsSource {
       *have = std::min<uint64_t>(need, SCRATCH_BYTES - SCRATCH_WS);
       return P0K_OK;
     }
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    HIPCHK(hipStreamIsCapturing(c->stream, &cs), "hipStreamIsCapturing");
-    if (cs != hipStreamCaptureStatusNone) {
-      std::lock_guard<std::mutex> lk(c->mu);
-      if (!c->own_capture) return P0K_OK;
-      if (need > c->ws_x_bytes) {
-        *out = c->ws_x;
-        *have = c->ws_x_bytes;
-        return P0K_OK;
-      }
+    bool capturing, ok;
+    if (int rr = ws_allowed(c, &capturing, &ok)) return rr;
+    if (!ok) return P0K_OK;
+    if (capturing && need > c->ws_x_bytes) {
+      *out = c->ws_x;
+      *have = c->ws_x_bytes;
+      return P0K_OK;
     }
     const int r = grow_ws(c, &c->ws_x, &c->ws_x_bytes, &c->ws_x_epoch, need, "prologue");
     if (r == P0K_OK) {
@@ -874,8 +871,8 @@ int p0k_attention(p0k_ctx *c, const p0k_attn_args *a) {
     tune = c->tune;
   }
   std::lock_guard<std::mutex> order(c->enq);
-  bool ws = true;
-  if (int rr = ws_allowed(c, &ws)) return rr;
+  bool capturing, ws;
+  if (int rr = ws_allowed(c, &capturing, &ws)) return rr;
   const unsigned runs = tune.attn_bq ? 0u : p0k::attention_runs(p, (int)tune.cus, ws, tune.attn_split);
   if (runs > 1) c->capture_ws = true;
   hipError_t e = p0k::launch_attention(p, (int)tune.cus, tune.attn_bq, runs, c->ws_attn, c->ws_attn_cnt, c->stream);
@@ -933,8 +930,9 @@ int p0k_graph_begin(p0k_ctx *c) {
   HIPCHK(hipSetDevice(c->device), "hipSetDevice");
   HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
   std::scoped_lock lk(c->enq, c->mu);
-  c->own_capture = true;
   c->capture_ws = false;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamGetCaptureInfo(c->stream, &cs, &c->own_capture) != hipSuccess) c->own_capture = 0;   // (its calls do without)
   return P0K_OK;
 }
 int p0k_graph_end(p0k_ctx *c, p0k_graph **out) {
@@ -946,7 +944,7 @@ int p0k_graph_end(p0k_ctx *c, p0k_graph **out) {
   {
     std::scoped_lock lk(c->enq, c->mu);
     ce = hipStreamEndCapture(c->stream, &g);
-    c->own_capture = false;
+    c->own_capture = 0;
     ws = c->capture_ws;
   }
   HIPCHK(ce, "hipStreamEndCapture");

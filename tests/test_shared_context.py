@@ -1,5 +1,6 @@
 """One context used by several threads, and graphs replayed through a context other than the one that captured them:
 calls that hand data from one launch to the next in the context's workspaces must not meet there (GPU)."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -107,3 +108,43 @@ def test_graph_launched_through_another_context(what):
     finally:
         own.close()
         other.close()
+
+
+def test_capture_ended_by_the_caller_is_forgotten():
+    """p0k_graph_begin's capture ended with the HIP API, then a capture begun by the caller: its attention call takes no
+    workspace (one run of keys: the bits of any other caller's capture, not those of the runs)."""
+    hip, dev = C.CDLL("libamdhip64.so"), p0k.Device(0)
+    s = C.c_void_p(p0k.lib().p0k_ctx_stream(dev.ctx))
+    rng = np.random.default_rng(6)
+    Hq, Hkv, Lk = 32, 8, 3777
+    q, k, v = (dev.upload(rng.standard_normal(n * 128).astype(np.float16)) for n in (Hq, Hkv * Lk, Hkv * Lk))
+    o = dev.buffer(Hq * 256)
+    a = {"q": {"buf": q}, "k": {"buf": k}, "v": {"buf": v}, "o": {"buf": o}, "Lq": 1, "Lk": Lk, "Hq": Hq, "Hkv": Hkv}
+
+    def captured():
+        graph, exe = C.c_void_p(), C.c_void_p()
+        dev.done()
+        assert hip.hipStreamBeginCapture(s, 1) == 0
+        try:
+            dev.attention(a)
+        finally:
+            assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+        assert hip.hipGraphLaunch(exe, s) == 0
+        got = dev.read(o, np.uint16, Hq * 128)
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)
+        return got
+
+    print("[p0k-test] a capture ended by the caller", flush=True)
+    try:
+        dev.attention(a)
+        runs, one = dev.read(o, np.uint16, Hq * 128), captured()
+        assert not np.array_equal(runs, one)
+        graph = C.c_void_p()
+        dev.graph_begin()
+        assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0
+        hip.hipGraphDestroy(graph)
+        assert np.array_equal(captured(), one)
+    finally:
+        dev.close()
