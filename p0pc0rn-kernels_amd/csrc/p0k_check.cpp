@@ -365,10 +365,12 @@ int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *e
   // N 4096 / 9216 / 28672 K 4096 13.6 / 45.6 / 61.8 -> 11.4 / 18.8 / 38.0, N 6144 K 14336 68.3 -> 31.5, N 4096 K 14336
   // 5 / 16 rows 34.3 / 36.8 -> 22.8 / 23.7, N 2048 K 1024 9.0 -> 6.5
   bool soft = false, xprep = false;
+  uint64_t soft_part = 0;
   if (kernel == K_GEMV_MF && we == P0K_ENC_F16 && (M >= 5 || K > gemv_sn_kmax(we)) && K >= 1024 && tune.gemv_mf < 0 && !tune.gemv_slices &&
       !tune.mfma_reg && tune.gemv_xprep != 0 && gemm_dma_ok(p, we, xm, wbytes) && (!xf32 || tune.decode_ws)) {
     kernel = K_MFMA;
     soft = xf32;
+    if (xf32 && S > 1) soft_part = (uint64_t)S * M * ((N + 127) / 128) * 512u;
     narrow = false;
   }
   // q4 / q8 on the matrix cores with fp32 rows: every item applies the prologue to its X again (and q8 then stages it
@@ -379,7 +381,7 @@ int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *e
     soft = xprep = true;
   if (out) *out = p;
   if (plan) {
-    plan->xprep = xprep; plan->soft = soft;
+    plan->xprep = xprep; plan->soft = soft; plan->soft_part = soft_part;
     plan->kernel = kernel; plan->we = we; plan->xm = xm; plan->bm = 16; plan->bn = kernel == K_GEMV_SN ? 16 : narrow ? 64 : 128; plan->mx = mx; plan->narrow = narrow;
     // the load-to-LDS kernel where it applies (P0K_MFMA_KERNEL=reg keeps the register-staged one, for tests)
     if (kernel == K_MFMA && gemm_dma_ok(p, we, xm, wbytes) && !tune.mfma_reg) kernel = plan->kernel = K_MFMA_DMA;

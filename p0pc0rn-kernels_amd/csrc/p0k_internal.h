@@ -10,8 +10,8 @@ enum { K_MFMA = 0, K_GEMV = 1, K_GEMV_MF = 2, K_MFMA_DMA = 3, K_GEMV_SN = 4 };
 // kernel choice of one call: GEMV items are (128-column tile) x (K slice of KS), S slices per tile
 // (load-to-LDS GEMM: S slices of K, wv waves, 0: by the tile)
 // (decode with fp32 rows: xprep, X' is materialised once; soft: a decode call that is planned with a workspace and has
-// another plan without, Tuning::decode_ws)
-struct Plan { int kernel, we, xm; unsigned bm, bn, S, KS; bool mx, narrow; unsigned wv; bool xprep, soft; };
+// another plan without, Tuning::decode_ws; soft_part: the partial sums that the plan without needs and this one does not)
+struct Plan { int kernel, we, xm; unsigned bm, bn, S, KS; bool mx, narrow; unsigned wv; bool xprep, soft; uint64_t soft_part; };
 // What the kernel choice depends on besides the call: the device's CU count and the P0K_* tuning switches of the
 // environment. A context reads them once (at creation and on p0k_ctx_reload_env); calls without a context read
 // them on the spot.

@@ -548,6 +548,18 @@ struct WsSource {
     (void)hipGetLastError();
     return P0K_OK;
   }
+  // make room for the partial sums of the plan that this call would have in a capture (which cannot grow them): a call
+  // outside a capture stands for the later one inside it
+  int reserve_part(uint64_t need) {
+    if (scratch || need >= (1ull << 32)) return P0K_OK;
+    bool capturing, ok;
+    if (int rr = ws_allowed(c, &capturing, &ok)) return rr;
+    if (capturing) return P0K_OK;
+    const int r = grow_ws(c, (void **)&c->ws_part, &c->ws_part_bytes, &c->ws_part_epoch, need, "decode");
+    if (r != P0K_E_NOMEM) return r;
+    (void)hipGetLastError();
+    return P0K_OK;
+  }
   // the X' workspace of a call that can do with less than `need`, or without: what there is of it, null where none can
   // be had (a caller captures the stream, nothing to grow during a capture, or no memory)
   int xws_if(uint64_t need, void **out, uint64_t *have) {
@@ -659,6 +671,8 @@ static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
     if (!xsoft || have < need) {
       tune.decode_ws = false;
       if ((r = p0k::prepare_gemm(a, &p, &plan, &err, tune))) return set_err(r, err);
+    } else if (int rr = ws.reserve_part(plan.soft_part)) {
+      return rr;
     }
   }
   {

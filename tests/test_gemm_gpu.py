@@ -305,6 +305,42 @@ def test_decode_rows_materialised(dev, kw, xprep, monkeypatch):
         own.close()
 
 
+# decode calls whose plan outside a capture differs from the one inside a caller's own (which takes no X' workspace)
+@pytest.mark.parametrize("kw", [dict(enc="f16", xmode="rms", epi="f16", M=8, N=512, K=4096),
+                                dict(enc="f16", xmode="lnmod", epi="resadd", M=1, N=256, K=9216),
+                                dict(enc="q8g64s.t64", xmode="rms", epi="f16", M=12, N=512, K=4096)],
+                         ids=lambda k: f"{k['enc']}-{k['xmode']}-M{k['M']}-K{k['K']}")
+def test_decode_captured_by_the_caller_after_one_call(kw):
+    """One call of a shape outside a capture is enough for a caller to capture that shape, on a context that made no other."""
+    c = make_case(seed=96, wscale=0.02, **kw)
+    banner(f"caller's capture after one call {kw}")
+    dev, hip = p0k.Device(0), C.CDLL("libamdhip64.so")
+    s = C.c_void_p(p0k.lib().p0k_ctx_stream(dev.ctx))
+    out = c.bufs[c.out]
+    try:
+        d = {k: dev.upload(v) for k, v in c.bufs.items()}
+        a = c.args(lambda n: d[n])
+        want = c.run_oracle(weights=oracle.CPU_WEIGHTS)
+        dev.gemm(a)
+        assert_close(dev.read(d[c.out], out.dtype, out.size), want, fp16=out.dtype == np.uint16, what="outside")
+        dev.upload(out, d[c.out])
+        graph, exe = C.c_void_p(), C.c_void_p()
+        assert hip.hipStreamBeginCapture(s, 1) == 0
+        try:
+            dev.gemm(a)
+        finally:
+            assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+        for _ in range(3):
+            dev.upload(out, d[c.out])
+            assert hip.hipGraphLaunch(exe, s) == 0
+            assert_close(dev.read(d[c.out], out.dtype, out.size), want, fp16=out.dtype == np.uint16, what="captured")
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)
+    finally:
+        dev.close()
+
+
 # ------------------------------------------------------------------------------------------------ dequantisation
 def _adversarial_q4(rows, K, seed):
     """random codes with (scale, min) words that include far-apart exponents (the decoder's exact-fp32 path)."""
