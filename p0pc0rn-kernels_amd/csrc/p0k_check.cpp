@@ -387,14 +387,14 @@ int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *e
     if (kernel == K_MFMA && gemm_dma_ok(p, we, xm, wbytes) && !tune.mfma_reg) kernel = plan->kernel = K_MFMA_DMA;
     plan->S = S; plan->KS = KS; plan->wv = 0;
     if (kernel == K_MFMA_DMA) {
-      // the X' that the call materialises (fp32 rows, GroupNorm): it shares the workspace room with the partial sums
+      // the X' that the call materialises (fp32 rows): it shares the workspace room with the partial sums
       const int xg = xm == P0K_X_CONV3 ? X_CONV3 : xm == P0K_X_CONV ? X_CONV : X_F16;
-      const uint64_t xbytes = xf32 ? (uint64_t)M * K * 2u : (f & F_GN) ? (uint64_t)p.nvox * p.Ci * 2u : 0u;
+      const uint64_t xbytes = xf32 ? (uint64_t)M * K * 2u : 0u;
       DmaPlan d;
       dma_plan(M, N, K, we, xg, xbytes, tune.cus, &d);
       // tuning / test override of the tile (P0K_MFMA_TILE=256x128, unsplit; results do not depend on it) and the slices
       if (tune.tile_m && dma_tile_ok(we, xg, tune.tile_m, tune.tile_n, tune.tile_wv)) d = DmaPlan{tune.tile_m, tune.tile_n, tune.tile_wv, 1};
-      if (tune.split && xg != X_CONV3 && d.bn == 128) {
+      if (tune.split && xg == X_F16 && d.bn == 128) {
         d.slices = std::min(tune.split, K / 64u);
         if (d.slices > 1 && xbytes + (uint64_t)d.slices * M * dma_ldp(N) * 4u > DMA_SPLIT_BYTES) d.slices = 1;
       }

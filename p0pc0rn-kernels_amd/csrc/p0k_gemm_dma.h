@@ -6,7 +6,7 @@
 // One workgroup computes a TBM x TBN tile (TBM, TBN in {128, 256}): 4 waves (2 x 2) for the smaller tiles, 8 waves
 // (2 x 4, two per SIMD, so one wave's decode and LDS reads run under the other's MFMAs) for 256 x 256 and, with f16
 // or q8 weights, 256 x 128; a wave owns (TBM/2) x (TBN/2), 128 x 64 or 128 x 32 as 32x32 v_mfma_f32_32x32x16_f16
-// blocks. For grids of few or short tiles, 8 waves lie 1 x 4 x 2 instead: a tile of any 32 rows x 128 columns, each wave
+// blocks. For grids of few or short tiles (not of convolutions), 8 waves lie 1 x 4 x 2 instead: a tile of any 32 rows x 128 columns, each wave
 // over all its rows and 32 columns, the two halves of the waves on alternate 64-k steps (WK = 2: a stage is two steps),
 // whose sums meet in LDS; and K may be cut into slices over workgroups (SPLIT), whose fp32 sums k_split_epi adds in slice
 // order before the epilogue. A weight is then decoded once per workgroup (2 x 4 decodes it in both row halves), the
@@ -188,6 +188,7 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
   constexpr int S = T::S, BI = T::BI, BJ = T::BJ, NW = T::NW;
   constexpr int WTM = T::WTM, WTN = T::WTN;
   constexpr bool HALF = XG == X_CONV3H, C3 = XG == X_CONV3 || HALF;
+  constexpr bool NAT = HALF || (XG == X_CONV && WE == W_F16);   // k of a step in the register-staged kernel's order
   static_assert(!HALF || (WE == W_F16 && WK == 1 && !SPLIT), "half steps: f16 weights, one order of K");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[T::SMEM];
 
@@ -356,9 +357,10 @@ __attribute__((amdgpu_waves_per_eu((DT<WE, TBM, TBN, NWV, WGM, WK>::OCC), (DT<WE
 #pragma unroll
     for (int j = 0; j < BJ; j++) rodd |= (wrow(p, nB + wn * WTN + 32 * j + l32) & 1u) << j;
   }
-  // the 8 k of a lane in 16-k sub-step `sub` (chunk of the step; hh: the lane's half). HALF keeps the register-staged
-  // kernel's order, the other path of these calls, so both give the same bits
-  auto chunk = [&](int sub) __attribute__((always_inline)) { return HALF ? 2 * sub + hh : 4 * hh + sub; };
+  // the 8 k of a lane in 16-k sub-step `sub` (chunk of the step; hh: the lane's half). NAT keeps the register-staged
+  // kernel's order, the other path of these calls, so both give the same bits (quantised weights: a lane's sub-steps are
+  // the words of one record)
+  auto chunk = [&](int sub) __attribute__((always_inline)) { return NAT ? 2 * sub + hh : 4 * hh + sub; };
   auto rdA_frag = [&](f16x8 *F, int st, int sub) __attribute__((always_inline)) {
     const uint8_t *sp = smem + st * T::STAGE + own + rdA + ((chunk(sub) ^ sw) & 7) * 16;
 #pragma unroll
@@ -674,14 +676,14 @@ hipError_t launch_dma_we(const Params &p, unsigned bm, unsigned bn, unsigned wv,
   if (bm == 256 && wv == 8) return launch_dma_one<WE, XG, 256, 128, 8, GM>(p, s);
   if (bm == 128 && wv == 8) return launch_dma_one<WE, XG, 128, 128, 8>(p, s);
   if (bm == 128 && wv == 4) return launch_dma_one<WE, XG, 128, 128>(p, s);
-  // (conv3 keeps one order of K, so it has no halves: its short tile is 2 x 4 waves of 32 x 32)
-  if constexpr (WE == W_F16 && (XG == X_CONV3 || XG == X_CONV3H)) {
+  // (the convolutions keep one order of K, so they have no halves: their short tile is 2 x 4 waves of 32 x 32)
+  if constexpr (WE == W_F16 && XG != X_F16) {
     if (bm == 64) return launch_dma_one<WE, XG, 64, 128, 8>(p, s);
   }
   if constexpr (WE == W_Q4) {
     if (bm == 256 && wv == 4) return launch_dma_one<WE, XG, 256, 128, 4>(p, s);
   }
-  if constexpr (XG != X_CONV3 && XG != X_CONV3H) {
+  if constexpr (XG == X_F16) {
     // wv == 2: 8 waves as 1 x 4 over the columns x 2 over K, any 32 rows
     switch (bm) {
     case 32: return launch_dma_one<WE, XG, 32, 128, 8, 1, 2, true>(p, s);

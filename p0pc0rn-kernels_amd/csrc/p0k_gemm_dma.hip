@@ -176,7 +176,7 @@ void dma_tile(uint32_t M, uint32_t N, int we, int xg, unsigned cus, unsigned *bm
 static unsigned dma_tall(int we) { return we == W_Q4 ? 256u : we == W_Q8 ? 224u : 192u; }
 
 bool dma_tile_ok(int we, int xg, unsigned bm, unsigned bn, unsigned wv) {
-  if (xg == X_CONV3) return wv != 2 && ((bm % 128 == 0 && bm <= 256) || (bm == 64 && bn == 128 && we == W_F16));
+  if (xg != X_F16) return wv != 2 && ((bm % 128 == 0 && bm <= 256) || (bm == 64 && bn == 128 && we == W_F16));
   if (bn == 256) return bm == 128 || bm == 256;
   if (bn != 128 || bm % 32 || bm < 32 || bm > 256) return false;
   return bm % 128 == 0 && wv != 2 ? true : bm <= dma_tall(we);
@@ -188,11 +188,11 @@ bool dma_tile_ok(int we, int xg, unsigned bm, unsigned bn, unsigned wv) {
 //   rounds of workgroups x (steps x (time of a 64-k step, less where the round leaves CUs idle) + fixed) (+ the slices'
 //   exchange),
 // whose constants are fitted to timed calls (q4, q8 and f16: 250-270 shapes each of 17..2048 rows x 1024..28672 columns x
-// K 1024..14336, convolutions: 36, every tile and 1..8 slices; rms 5-7 %; over those shapes the picks are 1-1.7 % above
-// the best and 1.8 times as fast as dma_tile's). Taken where it is 10 % under the estimate of dma_tile's tile, so that
+// K 1024..14336, every tile and 1..8 slices; rms 5-7 %; over those shapes the picks are 1-1.7 % above the best and 1.8
+// times as fast as dma_tile's). Taken where it is 10 % under the estimate of dma_tile's tile, so that
 // the fit's errors do not pick a slower one. us, before -> after: q4 17 x 4096 x 4096 40.6 -> 11.0, 77 x 6144 x 4096
 // 40.3 -> 16.8, 300 x 4096 x 14336 130 -> 48, 300 x 28672 x 4096 117 -> 88, 1000 x 4096 x 4096 55 -> 45; f16 77 x 6144 x
-// 4096 42.9 -> 16.5; 3x3 convolutions 64 x 64 x 512 -> 512 75.6 -> 38.8, 16 x 16 x 512 -> 512 66.8 -> 15.6.
+// 4096 42.9 -> 16.5.
 struct TileCost { unsigned m, n, wgs; double step, fix, idle; };
 struct SliceCost { double step[8], idle, fix, fix_row, split, split_mb; };   // step: of 32, 64 .. 256 rows
 static double rounds_us(uint64_t wgs, uint64_t slots, double steps, double step, double idle, double fix) {
@@ -201,31 +201,33 @@ static double rounds_us(uint64_t wgs, uint64_t slots, double steps, double step,
 }
 
 void dma_plan(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbytes, unsigned cus, DmaPlan *d) {
-  static const TileCost tiles[4][4] = {
+  static const TileCost tiles[3][4] = {
       {{128, 128, 1, 0.699, 5.32, 0.724}, {256, 128, 1, 1.143, 8.37, 0.375}, {256, 256, 1, 2.016, 13.3, 0.245}, {}},
       {{128, 128, 2, 0.869, 4.96, 0.630}, {256, 128, 1, 1.000, 6.70, 0.530}, {256, 256, 1, 1.855, 14.2, 0.357}, {}},
-      {{128, 128, 1, 0.521, 3.63, 0.539}, {128, 256, 1, 0.734, 8.52, 0.685}, {256, 128, 1, 0.824, 6.25, 0.506}, {256, 256, 1, 1.708, 13.4, 0.547}},
-      {{128, 128, 1, 0.593, 8.59, 0.831}, {128, 128, 2, 1.170, 10.3, 0.673}, {256, 128, 1, 1.079, 11.3, 0.719}, {}}};
-  static const SliceCost slices[4] = {
+      {{128, 128, 1, 0.521, 3.63, 0.539}, {128, 256, 1, 0.734, 8.52, 0.685}, {256, 128, 1, 0.824, 6.25, 0.506}, {256, 256, 1, 1.708, 13.4, 0.547}}};
+  static const SliceCost slices[3] = {
       {{0.308, 0.374, 0.443, 0.512, 0.609, 0.743, 0.831, 0.910}, 0.670, 2.70, 0.020, 2.54, 0.359},
       {{0.278, 0.336, 0.410, 0.503, 0.711, 0.785, 0.851, 0.0}, 0.644, 2.77, 0.027, 2.49, 0.364},
-      {{0.262, 0.326, 0.536, 0.608, 0.697, 0.761, 0.0, 0.0}, 0.689, 1.77, 0.024, 3.13, 0.341},
-      {{0.289, 0.362, 0.616, 0.695, 0.821, 0.918, 0.0, 0.0}, 0.846, 6.27, 0.026, 2.34, 0.428}};   // f16, the 2-D gather
+      {{0.262, 0.326, 0.536, 0.608, 0.697, 0.761, 0.0, 0.0}, 0.689, 1.77, 0.024, 3.13, 0.341}};
   d->wv = 0;
   d->slices = 1;
   dma_tile(M, N, we, xg, cus, &d->bm, &d->bn);
   const uint32_t nk = (K + DBK - 1) / DBK;
   // (K of a few steps is all fixed cost; quantised convolution weights were not timed)
   if (M == 0 || N == 0 || nk < 8 || (xg != X_F16 && we != W_F16)) return;
-  if (xg == X_CONV3) {
-    // one order of K whatever the clip (no halves, no slices): tiles of 64 and 128 rows x 128 with 8 waves for clips of few
-    // tiles, the same estimate (61 shapes, rms 2-5 %, picks within 0.5 % of the best). us, before -> after: 128 -> 128
-    // 32 x 32 51.3 -> 23.8, 3 x 41 x 123 52.5 -> 27.9, 2 x 92 x 160 53.1 -> 40.6; 256 -> 256 2 x 27 x 101 92.9 -> 46.0
-    static const TileCost c3[4] = {{256, 128, 1, 0.956, 8.14, 0.779}, {128, 128, 2, 1.301, 3.22, 0.613},
-                                   {128, 128, 1, 0.631, 4.45, 0.825}, {64, 128, 1, 0.403, 2.70, 0.857}};
+  if (xg != X_F16) {
+    // one order of K whatever the clip or the image (no halves, no slices): tiles of 64 and 128 rows x 128 with 8 waves for
+    // calls of few tiles, the same estimate (conv3 61 shapes, 2-D 44, rms 2-5 %, picks within 0.5 % of the best on average).
+    // us, before -> after: conv3 128 -> 128 32 x 32 51.3 -> 23.8, 3 x 41 x 123 52.5 -> 27.9, 2 x 92 x 160 53.1 -> 40.6; 256 ->
+    // 256 2 x 27 x 101 92.9 -> 46.0; 2-D 512 -> 512 64 x 64 73.7 -> 36.1, 16 x 16 58.2 -> 29.4 (slices of K gave 34.1 and
+    // 12.7, but an image taken in bands then had other bits than the whole one)
+    static const TileCost conv[2][4] = {{{256, 128, 1, 0.956, 8.14, 0.779}, {128, 128, 2, 1.301, 3.22, 0.613},
+                                         {128, 128, 1, 0.631, 4.45, 0.825}, {64, 128, 1, 0.403, 2.70, 0.857}},
+                                        {{256, 128, 1, 0.983, 8.76, 0.729}, {128, 128, 2, 1.269, 6.69, 0.547},
+                                         {128, 128, 1, 0.621, 5.99, 0.781}, {64, 128, 1, 0.404, 4.39, 0.848}}};
     const unsigned had = dma_wgs(we, d->bm, d->bn, 1, cus);
     double best = 0.0;
-    for (const TileCost &c : c3) {
+    for (const TileCost &c : conv[xg == X_CONV]) {
       const bool old = c.m == d->bm && c.n == d->bn && c.wgs == had;
       const double us = (old ? 0.95 : 1.0) * rounds_us((uint64_t)((M + c.m - 1) / c.m) * ((N + 127) / 128), (uint64_t)cus * c.wgs, nk,
                                                        c.step, c.idle, c.fix);
@@ -233,7 +235,7 @@ void dma_plan(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbyte
     }
     return;
   }
-  const int ei = xg == X_CONV ? 3 : we == W_Q4 ? 0 : we == W_Q8 ? 1 : 2;
+  const int ei = we == W_Q4 ? 0 : we == W_Q8 ? 1 : 2;
   const uint64_t tn = (N + 127) / 128, had = (uint64_t)((M + d->bm - 1) / d->bm) * ((N + d->bn - 1) / d->bn);
   const unsigned wgs = dma_wgs(we, d->bm, d->bn, had, cus);
   double best = 0.0;
@@ -261,7 +263,7 @@ void dma_plan(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbyte
 static hipError_t launch_dma_x(const Params &p, int we, int xg, unsigned bm, unsigned bn, unsigned wv, unsigned cus,
                                hipStream_t s) {
   const uint64_t tiles = (uint64_t)((p.M - p.mbase + bm - 1) / bm) * ((p.N - p.nbase + bn - 1) / bn);
-  if (!wv && bn == 128 && bm % 128) wv = xg == X_CONV3 ? 8 : 2;
+  if (!wv && bn == 128 && bm % 128) wv = xg != X_F16 ? 8 : 2;
   if (!wv) wv = dma_wgs(we, bm, bn, tiles, cus) == 1 ? 8 : 4;
   switch (we) {
   case W_Q4: return launch_dma_q4(p, xg, bm, bn, wv, s);

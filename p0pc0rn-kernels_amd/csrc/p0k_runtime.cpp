@@ -596,7 +596,7 @@ struct WsSource {
 // workspace, and the gather reads plain fp16 pixels (the register-staged kernel applies them once per tap and column
 // tile). A workspace smaller than the image takes it in bands of output rows, each with the input rows that its taps
 // touch (the K order, and so the bits, do not change); without room for one output row, the register-staged kernel.
-static hipError_t conv_gn(const p0k::Params &p0, const p0k::Plan &plan, p0k::DmaPlan d, const p0k::Tuning &tune, WsSource &ws,
+static hipError_t conv_gn(const p0k::Params &p0, const p0k::Plan &plan, const p0k::DmaPlan &d, const p0k::Tuning &tune, WsSource &ws,
                           int *err) {
   p0k::Params p = p0;
   const uint64_t line = (uint64_t)p.Wi * p.Ci * 2u;                 // bytes of an input row
@@ -612,11 +612,6 @@ static hipError_t conv_gn(const p0k::Params &p0, const p0k::Plan &plan, p0k::Dma
     unsigned bm, bn;
     p0k::mfma_tile(p.M, p.N, tune.cus, &bm, &bn);
     return p0k::launch_gemm_mfma(p, plan.we, plan.xm, bm, bn, ws.c->stream);
-  }
-  if (band < rows && d.slices > 1) {                                // (partial sums are rows of the whole call)
-    d = p0k::DmaPlan{0, 0, 0, 1};
-    p.slices = 1;
-    p0k::dma_tile(p.M, p.N, plan.we, p0k::X_CONV, tune.cus, &d.bm, &d.bn);
   }
   for (uint64_t y0 = 0; y0 < rows; y0 += band) {
     const uint64_t y1 = std::min<uint64_t>(rows, y0 + band);
@@ -694,15 +689,14 @@ static int gemm_run(p0k_ctx *c, const p0k_gemm_args *a, WsSource ws) {
   hipError_t e;
   p0k::DmaPlan d{plan.bm, plan.bn, plan.wv, plan.S};
   if (plan.kernel == p0k::K_MFMA_DMA && d.slices > 1) {
-    const uint64_t xbytes = plan.xm == P0K_X_CONV ? (p.flags & p0k::F_GN ? (uint64_t)p.nvox * p.Ci * 2u : 0u)
-                                                  : (plan.xm != P0K_X_F16 ? (uint64_t)a->M * a->K * 2u : 0u);
+    const uint64_t xbytes = plan.xm != P0K_X_F16 ? (uint64_t)a->M * a->K * 2u : 0u;
     p.ldp = p0k::dma_ldp(a->N);
     if (int rr = ws.slices_if(xbytes, (uint64_t)d.slices * a->M * p.ldp * sizeof(float), &p.part)) return rr;
     if (p.part) {
       p.slices = d.slices;
     } else {
       d = p0k::DmaPlan{0, 0, 0, 1};
-      p0k::dma_tile(a->M, a->N, plan.we, plan.xm == P0K_X_CONV ? p0k::X_CONV : p0k::X_F16, tune.cus, &d.bm, &d.bn);
+      p0k::dma_tile(a->M, a->N, plan.we, p0k::X_F16, tune.cus, &d.bm, &d.bn);
     }
   }
   if (plan.kernel == p0k::K_GEMV_SN) {
