@@ -63,7 +63,7 @@ Tuning tuning_from_env(unsigned cus) {
   if (const char *ov = getenv("P0K_MFMA_KERNEL")) t.mfma_reg = strcmp(ov, "reg") == 0;
   if (const char *ov = getenv("P0K_MFMA_TILE")) {
     unsigned tm = 0, tn = 0, wv = 0;
-    if (sscanf(ov, "%ux%ux%u", &tm, &tn, &wv) >= 2 && dma_tile_ok(P0K_ENC_Q4G32A_T64, X_F16, tm, tn, wv)) {
+    if (sscanf(ov, "%ux%ux%u", &tm, &tn, &wv) >= 2 && (tn == 128 || (tn == 256 && tm % 128 == 0)) && tm % 32 == 0 && tm && tm <= 256) {
       t.tile_m = tm;
       t.tile_n = tn;
       t.tile_wv = wv == 2 || wv == 4 || wv == 8 ? wv : 0;
@@ -392,12 +392,7 @@ int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *e
       const uint64_t xbytes = xf32 ? (uint64_t)M * K * 2u : 0u;
       DmaPlan d;
       dma_plan(M, N, K, we, xg, xbytes, tune.cus, &d);
-      // tuning / test override of the tile (P0K_MFMA_TILE=256x128, unsplit; results do not depend on it) and the slices
-      if (tune.tile_m && dma_tile_ok(we, xg, tune.tile_m, tune.tile_n, tune.tile_wv)) d = DmaPlan{tune.tile_m, tune.tile_n, tune.tile_wv, 1};
-      if (tune.split && xg == X_F16 && d.bn == 128) {
-        d.slices = std::min(tune.split, K / 64u);
-        if (d.slices > 1 && xbytes + (uint64_t)d.slices * M * dma_ldp(N) * 4u > DMA_SPLIT_BYTES) d.slices = 1;
-      }
+      dma_forced(M, N, K, we, xg, xbytes, tune, &d);
       plan->bm = d.bm; plan->bn = d.bn; plan->wv = d.wv; plan->S = d.slices;
     }
     if (kernel == K_MFMA) {

@@ -674,7 +674,9 @@ hipError_t launch_dma_we(const Params &p, unsigned bm, unsigned bn, unsigned wv,
   }
   if (bn != 128) return hipErrorInvalidValue;
   if (bm == 256 && wv == 8) return launch_dma_one<WE, XG, 256, 128, 8, GM>(p, s);
-  if (bm == 128 && wv == 8) return launch_dma_one<WE, XG, 128, 128, 8>(p, s);
+  if constexpr (WE != W_Q8) {
+    if (bm == 128 && wv == 8) return launch_dma_one<WE, XG, 128, 128, 8>(p, s);
+  }
   if (bm == 128 && wv == 4) return launch_dma_one<WE, XG, 128, 128>(p, s);
   // (the convolutions keep one order of K, so they have no halves: their short tile is 2 x 4 waves of 32 x 32)
   if constexpr (WE == W_F16 && XG != X_F16) {

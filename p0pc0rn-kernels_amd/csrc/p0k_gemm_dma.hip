@@ -1,6 +1,7 @@
 // p0k_gemm_dma.hip — the host side of the load-to-LDS GEMM (p0k_gemm_dma.h): which calls qualify, the tile and the split
 // of a call, and the passes that materialise X' once per element.
 #include "p0k_gemm_dma.h"
+#include "p0k_internal.h"
 
 namespace p0k {
 
@@ -175,11 +176,29 @@ void dma_tile(uint32_t M, uint32_t N, int we, int xg, unsigned cus, unsigned *bm
 // the tallest tile of the 1 x 4 x 2 wave layout: two stages of two steps within 160 KB
 static unsigned dma_tall(int we) { return we == W_Q4 ? 256u : we == W_Q8 ? 224u : 192u; }
 
+// the instances of launch_dma_we
 bool dma_tile_ok(int we, int xg, unsigned bm, unsigned bn, unsigned wv) {
-  if (xg != X_F16) return wv != 2 && ((bm % 128 == 0 && bm <= 256) || (bm == 64 && bn == 128 && we == W_F16));
-  if (bn == 256) return bm == 128 || bm == 256;
-  if (bn != 128 || bm % 32 || bm < 32 || bm > 256) return false;
-  return bm % 128 == 0 && wv != 2 ? true : bm <= dma_tall(we);
+  if (bn == 256) return wv == 0 && (bm == 128 || bm == 256);
+  if (bn != 128) return false;
+  switch (wv) {
+  case 0: return bm == 128 || bm == 256;                                   // (4 or 8 waves, as dma_wgs says)
+  case 2: return xg == X_F16 && bm % 32 == 0 && bm != 0 && bm <= dma_tall(we);
+  case 4: return bm == 128 || (bm == 256 && we == W_Q4);
+  case 8: return bm == 256 || (bm == 128 && we != W_Q8) || (bm == 64 && we == W_F16 && xg != X_F16);
+  }
+  return false;
+}
+
+void dma_forced(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbytes, const Tuning &t, DmaPlan *d) {
+  for (unsigned wv : {t.tile_wv, 0u, 2u, 8u})
+    if (t.tile_m && dma_tile_ok(we, xg, t.tile_m, t.tile_n, wv)) {
+      *d = DmaPlan{t.tile_m, t.tile_n, wv, 1};
+      break;
+    }
+  if (t.split && d->bn == 128 && dma_tile_ok(we, xg, d->bm, 128, 2)) {
+    d->slices = t.split < K / DBK ? t.split : K / DBK;
+    if (d->slices > 1 && xbytes + (uint64_t)d->slices * M * dma_ldp(N) * 4u > DMA_SPLIT_BYTES) d->slices = 1;
+  }
 }
 
 // The plan of a call: dma_tile's tile; or, for grids that leave it idle or tiles half empty, a tile of the 1 x 4 x 2 wave

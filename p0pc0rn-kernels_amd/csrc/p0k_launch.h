@@ -27,8 +27,12 @@ hipError_t launch_xprep(const Params &p, int xm, uint16_t *xp, hipStream_t s);
 // the plan of a load-to-LDS call: tile, waves (0: as dma_wgs says), slices of K
 struct DmaPlan { unsigned bm, bn, wv, slices; };
 constexpr uint64_t DMA_SPLIT_BYTES = 31ull << 20;   // X' and partial sums of a split call at most (the scratch array's room)
-bool dma_tile_ok(int we, int xg, unsigned bm, unsigned bn, unsigned wv);   // a tile of the load-to-LDS kernel
+bool dma_tile_ok(int we, int xg, unsigned bm, unsigned bn, unsigned wv);   // there is such a load-to-LDS kernel
 void dma_plan(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbytes, unsigned cus, DmaPlan *d);
+// the tuning / test overrides of a plan (P0K_MFMA_TILE, P0K_MFMA_SPLIT): the tile unsplit, with its own wave layout where it
+// has no kernel with the one asked for; slices of K where the plan's tile has them. What no kernel has leaves the plan alone
+struct Tuning;
+void dma_forced(uint32_t M, uint32_t N, uint32_t K, int we, int xg, uint64_t xbytes, const Tuning &t, DmaPlan *d);
 inline uint32_t dma_ldp(uint32_t N) { return (N + 127u) / 128u * 128u; }   // row length of the partial sums
 // cus: the device's CU count; tail: allow the column split of dma_tail. p.slices > 1: p.part holds slices * M * ldp floats
 hipError_t launch_gemm_dma(const Params &p, int we, int xg, const DmaPlan &d, unsigned cus, bool tail, hipStream_t s);

@@ -780,6 +780,41 @@ def test_every_mfma_tile_matches_oracle(dev, kw, kernel, monkeypatch):
         assert np.array_equal(o, outs[0])
 
 
+@pytest.mark.parametrize("enc", ["q4g32a.t64", "q8g64s.t64", "f16"])
+@pytest.mark.parametrize("kind", ["rows", "conv", "conv3"])
+def test_every_documented_tile_and_split_runs(dev, enc, kind, monkeypatch):
+    """P0K_MFMA_TILE with every wave layout and P0K_MFMA_SPLIT over all that they take: a combination that no kernel has
+    leaves the planner's choice, none is an error, and every result matches the oracle."""
+    if kind == "rows":
+        c = make_case(enc=enc, epi="f16", M=290, N=200, K=512, seed=37)
+    elif kind == "conv":
+        c = make_conv2d_case(Hi=17, Wi=18, Ci=64, N=192, enc=enc)
+    else:
+        c = make_conv3_case(T=2, H=9, W=17, C=64, N=192, enc=enc)
+    d = {k: dev.upload(v) for k, v in c.bufs.items()}
+    a, y = c.args(lambda n: d[n]), c.bufs["y"]
+    want = c.run_oracle(weights=oracle.KERNEL_WEIGHTS)
+    try:
+        for t in [f"{m}x{n}" for n in (128, 256) for m in range(32, 257, 32)]:
+            banner(f"{enc} {kind} tile {t}")
+            for w in ("", "x2", "x4", "x8"):
+                monkeypatch.setenv("P0K_MFMA_TILE", t + w)
+                for split in ("0", "1", "3"):
+                    monkeypatch.setenv("P0K_MFMA_SPLIT", split)
+                    dev.upload(np.zeros_like(y), d["y"])
+                    dev.gemm(a)
+                    assert_close(dev.read(d["y"], np.uint16, y.size), want, what=f"tile {t}{w} split {split}")
+        monkeypatch.delenv("P0K_MFMA_TILE")
+        for split in ("1", "2", "8"):
+            monkeypatch.setenv("P0K_MFMA_SPLIT", split)
+            dev.upload(np.zeros_like(y), d["y"])
+            dev.gemm(a)
+            assert_close(dev.read(d["y"], np.uint16, y.size), want, what=f"planned tile, split {split}")
+    finally:
+        for b in d.values():
+            dev.free(b)
+
+
 # epilogues that read Y: whole 16-byte groups, a ragged last group beside whole ones, and rows or bases off that alignment
 RESIDUAL_CASES = [
     dict(enc="q4g32a.t64", xmode="rms", epi="resadd", M=301, N=204, ld_pad=4, K=192, gate=True),
