@@ -105,16 +105,16 @@ static bool sn_rule(int we, uint32_t N, uint32_t K, uint32_t M, unsigned cus) {
   return M <= 2 && K <= 8192u && items * 2u <= (uint64_t)cus * (M == 1 ? 3u : 2u);
 }
 
-// Where the matrix-core decode of q4 / q8 gets its rms / lnmod rows materialised by a pass of their own (about 3 us with
-// its launch). us, in every item -> by the pass: q8 (whose fp16 rows stream with the weights; the fused form stages X' of
-// the item behind a barrier) N 4096 K 4096 5 / 16 rows 14.3 / 26.0 -> 11.7 / 13.0, N 28672 K 4096 2 / 12 rows 23.9 / 33.1
-// -> 22.4 / 25.0, K 14336 18.6 -> 18.1 (5 rows), N 2048 K 1024 5 / 16 rows 7.1 / 9.4 -> 7.7 / 8.9; q4 N 28672 K 4096 5 rows
-// 24.1 -> 17.4, N 4096 K 4096 5 / 8 / 16 rows 12.2 / 12.8 / 15.0 -> 11.8 / 11.8 / 12.0, N 4096 K 2048 5 / 16 rows 8.1 /
-// 9.7 -> 8.4 / 8.8, N 4096 K 8192 12.6 -> 13.2 (not taken), N 6144 K 14336 21.3 -> 20.3; lnmod gains more.
-static bool xprep_rule(int we, uint32_t N, uint32_t K, uint32_t M) {
-  if (we == P0K_ENC_Q8G64S_T64) return K >= 2048u || (M >= 12u && K >= 1024u);
-  return (uint64_t)N * K >= 50u * 1000u * 1000u || (K <= 4096u && (uint64_t)M * K >= 32768u);
-}
+// Where the matrix-core decode of q4 / q8 gets its rms / lnmod rows materialised by a pass of their own: where an item's
+// range of K is long (KS; its share of K when K is split), since every item applies the prologue to that range of its rows
+// again and, with q8, stages it behind a barrier. 30 shapes (N 1024..28672, K 1024..14336) x 1..16 rows, weights from HBM:
+// KS 2048 and more gains nearly everywhere, 512 and less loses 0.5-2 us (the pass and its launch), 1024 gains but in 64-column
+// items of few rows; the picks are 0.1-0.2 % above the best on average, 5 % at most. us, in every item -> by the pass: q8 N
+// 4096 K 4096 6 / 16 rows 16.0 / 26.4 -> 12.4 / 14.1, heads at 1 / 16 rows (K in 8 slices) 12.9 / 14.6 -> 13.6 / 15.2 (not
+// taken); N 28672 K 4096 2 / 12 rows 26.0 / 35.3 -> 25.5 / 27.4; N 6144 K 1024 6 / 12 rows 7.5 / 8.7 -> 7.8 / 8.4; q4 N 28672
+// K 4096 5 rows 25.2 -> 18.8, N 4096 K 4096 5 / 16 rows 13.9 / 15.7 -> 12.6 / 13.0, its heads 11.9 / 12.6 -> 12.7 / 13.7 (not
+// taken), N 4096 K 14336 5 rows 17.2 -> 16.4.
+static bool xprep_rule(uint32_t KS, uint32_t M, bool narrow) { return KS > 1024u || (KS == 1024u && (M >= 9u || !narrow)); }
 
 int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *err, const Tuning &tune) {
   NEED(a != nullptr, "gemm: no arguments");
@@ -376,7 +376,7 @@ int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *e
   // q4 / q8 on the matrix cores with fp32 rows: every item applies the prologue to its X again (and q8 then stages it
   // instead of streaming it with the weights); materialised once, the decode reads fp16 rows
   if (kernel == K_GEMV_MF && xf32 && we != P0K_ENC_F16 && tune.decode_ws && tune.gemv_xprep != 0 &&
-      (tune.gemv_xprep == 1 || xprep_rule(we, N, K, M)) &&
+      (tune.gemv_xprep == 1 || xprep_rule(KS, M, narrow)) &&
       (uint64_t)M * K * 2u + (S > 1 ? (uint64_t)S * M * ((N + 127) / 128) * 512u : 0u) <= DMA_SPLIT_BYTES)
     soft = xprep = true;
   if (out) *out = p;

@@ -305,6 +305,33 @@ def test_decode_rows_materialised(dev, kw, xprep, monkeypatch):
         own.close()
 
 
+@pytest.mark.parametrize("enc,epi,M,N,K,taken", [
+    ("q8g64s.t64", "heads", 1, 4096, 4096, False), ("q8g64s.t64", "heads", 16, 4096, 4096, False), ("q8g64s.t64", "f16", 6, 512, 1024, False),
+    ("q8g64s.t64", "f16", 9, 512, 1024, True), ("q8g64s.t64", "f16", 12, 512, 4096, True), ("q8g64s.t64", "f16", 16, 512, 8192, False),
+    ("q4g32a.t64", "heads", 9, 1536, 4096, False), ("q4g32a.t64", "f16", 5, 512, 4096, True), ("q4g32a.t64", "f16", 16, 512, 8192, False)])
+def test_rows_materialised_where_an_item_has_a_long_range_of_k(enc, epi, M, N, K, taken, monkeypatch):
+    """The rule of the X' pass, seen in the workspaces of a context that made no other call: taken where an item's range of K
+    is 1024 and more (64-column items of 1024 from 9 rows on), not where the split of K leaves each item a short one."""
+    kw = dict(Hq=N // 128 - 2, Hkv=1) if epi == "heads" else {}
+    c = make_case(enc=enc, xmode="rms", epi=epi, M=M, N=N, K=K, seed=97, wscale=0.02, **kw)
+    banner(f"X' rule {enc} {epi} M={M} N={N} K={K}")
+    held = []
+    for sw in ("0", None):
+        if sw is None:
+            monkeypatch.delenv("P0K_GEMV_XPREP")
+        else:
+            monkeypatch.setenv("P0K_GEMV_XPREP", sw)
+        own = p0k.Device(0)
+        try:
+            got = c.run_device(own)
+            assert c.kernel == "gemv_mfma"
+            held.append(own.workspace_stats()["live_bytes"])
+        finally:
+            own.close()
+        assert_close(got, c.run_oracle(weights=oracle.CPU_WEIGHTS), what=f"P0K_GEMV_XPREP={sw}")
+    assert (held[1] > held[0]) == taken, held
+
+
 # decode calls whose plan outside a capture differs from the one inside a caller's own (which takes no X' workspace)
 @pytest.mark.parametrize("kw", [dict(enc="f16", xmode="rms", epi="f16", M=8, N=512, K=4096),
                                 dict(enc="f16", xmode="lnmod", epi="resadd", M=1, N=256, K=9216),
