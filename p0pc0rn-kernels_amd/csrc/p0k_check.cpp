@@ -116,6 +116,20 @@ static bool sn_rule(int we, uint32_t N, uint32_t K, uint32_t M, unsigned cus) {
 // taken), N 4096 K 14336 5 rows 17.2 -> 16.4.
 static bool xprep_rule(uint32_t KS, uint32_t M, bool narrow) { return KS > 1024u || (KS == 1024u && (M >= 9u || !narrow)); }
 
+// Where f16 weights with 5..16 rows, or fewer where K is past the short-call items, take the load-to-LDS GEMM's 32-row tile
+// instead of the matrix-core decode (fp16 products summed in fp32 in both): everywhere but where the decode's items fill the
+// CUs in one round with little to do each: K of 1024 in 64-column items, or, with rows that the GEMM would have to
+// materialise, K in 4..8 slices of at most 512. 954 calls (N 1024..28672, K 1024..14336, weights from HBM): 1.35 times as
+// fast on average, none slower than 1.014 of the decode, picks 0.01 % above the better side (2.7 % at most). us, decode -> GEMM,
+// 16 rows unless stated: N 4096 K 4096 / 8192 15.2 / 30.7 -> 15.0 / 20.9, N 28672 K 4096 68.5 -> 46.9, N 2048 K 1024 9.4 -> 7.3,
+// N 6144 K 14336 1 / 16 rows 63.5 / 70.1 -> 38.2 / 39.1, N 28672 K 1024 23.8 -> 14.4; not taken: N 14336 K 1024 5 rows 9.4 ->
+// 10.6, with rms 10.8 -> 13.0; rms N 6144 / 8192 K 1024 5 rows 10.6 / 10.9 -> 11.9 / 12.2, N 4096 K 4096 15.4 -> 17.3
+static bool f16_gemm_rule(bool xf32, uint32_t K, uint32_t S, uint32_t KS, bool narrow, uint32_t N, unsigned cus) {
+  const uint64_t items = (uint64_t)S * ((N + 127u) / 128u) * (narrow ? 2u : 1u);
+  if (narrow && K <= 1024u && items <= cus) return false;
+  return !(xf32 && S >= 4u && S <= 8u && KS <= 512u && 4u * items >= 3u * cus && items <= cus);
+}
+
 int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *err, const Tuning &tune) {
   NEED(a != nullptr, "gemm: no arguments");
   NEED(a->struct_size == sizeof(p0k_gemm_args), "gemm: struct_size %u, this library expects %u (ABI %d)", a->struct_size,
@@ -360,14 +374,11 @@ int prepare_gemm(const p0k_gemm_args *a, Params *out, Plan *plan, std::string *e
       }
     }
   }
-  // f16 weights, 5..16 rows, or fewer where K is past the short-call items: the load-to-LDS GEMM's 32-row tile reads them
-  // 1.2 to 2.5 times as fast as the matrix-core decode (fp16 products summed in fp32 in both). us, 16 rows unless stated:
-  // N 4096 / 9216 / 28672 K 4096 13.6 / 45.6 / 61.8 -> 11.4 / 18.8 / 38.0, N 6144 K 14336 68.3 -> 31.5, N 4096 K 14336
-  // 5 / 16 rows 34.3 / 36.8 -> 22.8 / 23.7, N 2048 K 1024 9.0 -> 6.5
   bool soft = false, xprep = false;
   uint64_t soft_part = 0;
   if (kernel == K_GEMV_MF && we == P0K_ENC_F16 && (M >= 5 || K > gemv_sn_kmax(we)) && K >= 1024 && tune.gemv_mf < 0 && !tune.gemv_slices &&
-      !tune.mfma_reg && tune.gemv_xprep != 0 && gemm_dma_ok(p, we, xm, wbytes) && (!xf32 || tune.decode_ws)) {
+      !tune.mfma_reg && tune.gemv_xprep != 0 && gemm_dma_ok(p, we, xm, wbytes) && (!xf32 || tune.decode_ws) &&
+      f16_gemm_rule(xf32, K, S, KS, narrow, N, tune.cus)) {
     kernel = K_MFMA;
     soft = xf32;
     if (xf32 && S > 1) soft_part = (uint64_t)S * M * ((N + 127) / 128) * 512u;

@@ -261,6 +261,19 @@ def test_short_decode_routing(monkeypatch):
     assert q8(2, 40960, 8192) == "gemv_short" and q8(1, 4096, 16384) != "gemv_short"
 
 
+def test_f16_decode_or_gemm_routing():
+    """f16 weights with 5..16 rows take the load-to-LDS GEMM, but not where the decode's items fill the CUs in one round with
+    little to do each: K of 1024 in 64-column items, or fp32 rows with K in 4..8 slices of at most 512."""
+    f16 = lambda M, N, K, **kw: p0k.select_tile(host_args(make_case(M=M, enc="f16", N=N, K=K, **kw)))["kernel"]   # noqa: E731
+    assert f16(5, 14336, 1024) == "gemv_mfma" and f16(16, 14336, 1024, xmode="rms") == "gemv_mfma"
+    assert f16(5, 18432, 1024) == "mfma_dma" and f16(8, 14336, 2048) == "mfma_dma"
+    for N, K in ((6144, 1024), (8192, 1024), (4096, 2048), (4096, 4096)):
+        assert f16(8, N, K, xmode="rms") == "gemv_mfma" and f16(8, N, K) == "mfma_dma"
+    for N, K in ((5120, 1024), (2048, 2048), (6144, 2048), (2048, 4096), (6144, 4096)):
+        assert f16(8, N, K, xmode="lnmod") == "mfma_dma"
+    assert f16(1, 256, 9216, xmode="rms") == "mfma_dma" and f16(1, 256, 9216) == "mfma_dma"
+
+
 def test_null_context_calls_are_refused():
     L = p0k.lib()
     assert L.p0k_ctx_reload_env(None) == p0k.E_ARG
