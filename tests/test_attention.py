@@ -90,7 +90,7 @@ def cos_and_err(got, want):
 @pytest.mark.parametrize("bq", [128, 256])
 @pytest.mark.parametrize("c", ATT + MORE, ids=lambda c: c["label"])
 def test_attention_matches_oracle(dev, c, bq, monkeypatch):
-    """Both workgroup sizes (128 / 256 queries) on every case; the library picks 256 only for large grids."""
+    """Both workgroup sizes on every case (the library takes 128 queries; 256 are a tuning switch)."""
     monkeypatch.setenv("P0K_ATTN_BQ", str(bq))
     print(f"attention bq={bq} {c}", flush=True)
     q, k, v = setup(c, 21, 1.0 if c.get("cap") else 0.5)
@@ -123,17 +123,22 @@ def test_attention_matches_oracle(dev, c, bq, monkeypatch):
 # Causal grids of more blocks than CUs, longest blocks first: heads a multiple of 8 (an XCD's own) and not, all blocks
 # resident at once (the second on each CU in the opposite order) and more, a valid length that levels the work
 @pytest.mark.gpu
-@pytest.mark.parametrize("Hq,Hkv,L,nvalid", [(40, 8, 900, 900), (35, 7, 1000, 990), (48, 6, 1500, 700), (72, 9, 513, 513)])
-def test_attention_causal_block_order(dev, Hq, Hkv, L, nvalid):
+# (cap: the soft-capped kernels; bq 256: the blocks of the tuning switch)
+@pytest.mark.parametrize("Hq,Hkv,L,nvalid,cap,bq", [(40, 8, 900, 900, 0, 0), (35, 7, 1000, 990, 0, 0), (48, 6, 1500, 700, 0, 0), (72, 9, 513, 513, 0, 0),
+                                                    (40, 8, 900, 880, 2.0, 0), (48, 6, 1500, 1500, 2.0, 0), (72, 9, 1000, 990, 0, 256), (35, 7, 2000, 1999, 2.0, 256)])
+def test_attention_causal_block_order(dev, Hq, Hkv, L, nvalid, cap, bq, monkeypatch):
     """Sampled rows of every head and block against float64 numpy, with the file's fp16 tolerance (every block of the
     grid computes some of them, so a block taken twice and another never would show)."""
-    print(f"causal order Hq={Hq} L={L} nvalid={nvalid}", flush=True)
+    print(f"causal order Hq={Hq} L={L} nvalid={nvalid} cap={cap} bq={bq}", flush=True)
+    if bq:
+        monkeypatch.setenv("P0K_ATTN_BQ", str(bq))
+    assert (L + (bq or 128) - 1) // (bq or 128) * Hq > dev.cus()
     c = dict(Hq=Hq, Hkv=Hkv, Lq=L, Lk=L, mode=1, nvalid=nvalid)
     q, k, v = setup(c, 23)
     bufs = [dev.upload(a) for a in (q, k, v)] + [dev.buffer(L * Hq * 256)]
     try:
         dev.attention({"q": {"buf": bufs[0]}, "k": {"buf": bufs[1]}, "v": {"buf": bufs[2]}, "o": {"buf": bufs[3]}, "Lq": L,
-                       "Lk": L, "Hq": Hq, "Hkv": Hkv, "mode": 1, "nvalid": nvalid})
+                       "Lk": L, "Hq": Hq, "Hkv": Hkv, "mode": 1, "nvalid": nvalid, "cap": cap})
         got = oracle.h2f(dev.read(bufs[3], np.uint16, L * Hq * 128)).reshape(L, Hq, 128)
     finally:
         for b in bufs:
@@ -142,6 +147,7 @@ def test_attention_causal_block_order(dev, Hq, Hkv, L, nvalid):
     rows = sorted({min(L - 1, 128 * b + o) for b in range((L + 127) // 128) for o in (0, 31, 127)})
     for h in range(Hq):
         s = Q[h, rows] @ K[h // (Hq // Hkv)].T / np.sqrt(128.0)
+        s = cap * np.tanh(s / cap) if cap else s
         s = np.where(np.arange(L)[None, :] <= np.minimum(np.array(rows), nvalid - 1)[:, None], s, -np.inf)
         p = np.exp(s - s.max(1, keepdims=True))
         want = (p / p.sum(1, keepdims=True)) @ V[h // (Hq // Hkv)]
@@ -212,6 +218,47 @@ def test_attention_few_queries(dev, c, how):
     err = np.abs(oracle.h2f(o[:, :Hq * 128].ravel()) - want)
     bound = 2 ** -8 * np.abs(want).max() + 2 ** -9 * np.abs(want)
     assert np.all(err <= bound), f"max err {err.max()} (bound {bound.max()})"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("split", ["0", "1"])
+@pytest.mark.parametrize("Lq,Lk,nvalid", [(1, 3000, 2500), (16, 700, 389), (40, 300, 200)])
+def test_attention_values_that_are_not_finite(dev, Lq, Lk, nvalid, split, monkeypatch):
+    """Both kernels. NaN in the cache past the last tile of 64 keys that the valid length reaches: not seen. Keys whose score
+    is -inf: as if they were not there. A key whose score is +inf: NaN, in every row that sees it."""
+    monkeypatch.setenv("P0K_ATTN_SPLIT", split)
+    print(f"not finite Lq={Lq} Lk={Lk} nvalid={nvalid} split={split}", flush=True)
+    c = dict(Hq=4, Hkv=2, Lq=Lq, Lk=Lk, mode=2, nvalid=nvalid)
+    rng = np.random.default_rng(Lk)
+    Q = np.abs(rng.standard_normal((4, Lq, 128)) * 0.5).astype(np.float16) + np.float16(0.01)     # (positive)
+    K = (rng.standard_normal((2, Lk, 128)) * 0.5).astype(np.float16)
+    V = rng.standard_normal((2, Lk, 128)).astype(np.float16)
+
+    def run(K, V):
+        bufs = [dev.upload(a) for a in (Q, K, V)] + [dev.buffer(Lq * 4 * 256)]
+        try:
+            dev.attention({"q": {"buf": bufs[0]}, "k": {"buf": bufs[1]}, "v": {"buf": bufs[2]}, "o": {"buf": bufs[3]}, **c})
+            return oracle.h2f(dev.read(bufs[3], np.uint16, Lq * 512)).reshape(Lq, 4, 128)
+        finally:
+            for b in bufs:
+                dev.free(b)
+
+    clean = run(K, V)
+    Kn, Vn = K.copy(), V.copy()
+    Kn[:, (nvalid + 63) // 64 * 64:] = Vn[:, (nvalid + 63) // 64 * 64:] = np.nan
+    assert np.array_equal(run(Kn, Vn), clean) and np.isfinite(clean).all()
+    gone = [0, 31, 32, 100, nvalid - 1]
+    Ki = K.copy()
+    Ki[:, gone] = -np.inf
+    keep = np.setdiff1d(np.arange(nvalid), gone)
+    want = numpy_attention(Q.view(np.uint16), np.ascontiguousarray(K[:, keep]).view(np.uint16), np.ascontiguousarray(V[:, keep]).view(np.uint16),
+                           dict(c, Lk=keep.size, mode=0)).reshape(Lq, 4, 128)
+    err = np.abs(run(Ki, V) - want)
+    assert np.all(err <= 2 ** -8 * np.abs(want).max() + 2 ** -9 * np.abs(want)), f"max err {err.max()}"
+    Kp = K.copy()
+    Kp[0, 150] = np.inf                                   # kv head 0: query heads 0 and 1
+    got = run(Kp, V)
+    assert np.isnan(got[:, :2]).all() and np.array_equal(got[:, 2:], clean[:, 2:])
 
 
 @pytest.mark.gpu
