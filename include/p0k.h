@@ -143,7 +143,8 @@ typedef struct p0k_gn_args {
  * i iff j <= min(i, nvalid - 1); 2: j < nvalid. GQA: query head h reads kv head h / (Hq / Hkv). Zero fields take the
  * reference's defaults: Lk = Lq, Hkv = Hq, nvalid = Lk, ldo = Hq * 128, scale = 1 / sqrt(128); cap > 0 soft-caps
  * the scores to cap * tanh(s / cap). A call with few query rows may divide its keys over workgroups through a fixed
- * workspace of the context (not in a capture begun by the caller, whose graph may replay on another stream). Offsets and sizes in bytes; q / k / v offsets 16-byte aligned, o 8-byte. */
+ * workspace of the context (not in a capture begun by the caller, whose graph may replay on another stream). Offsets and
+ * sizes in bytes; q / k / v offsets 16-byte aligned, o 8-byte. */
 typedef struct p0k_attn_args {
   uint32_t struct_size;
   const void *q_buf; uint64_t q_off, q_size;
@@ -177,7 +178,8 @@ int p0k_ctx_create(int device, p0k_ctx **out);
 void p0k_ctx_destroy(p0k_ctx *ctx);
 int p0k_device_info_get(p0k_ctx *ctx, p0k_device_info *out);
 /* Kernel choice reads the device's CU count and the P0K_* tuning switches of the environment (P0K_MFMA_TILE,
- * P0K_MFMA_KERNEL, P0K_DMA_TAIL, P0K_GEMV_MF, P0K_GEMV_MQ4, P0K_GEMV_SLICES, P0K_GEMV_XPREP, P0K_MFMA_SPLIT, P0K_ATTN_BQ, P0K_ATTN_SPLIT) once, when the context is created;
+ * P0K_MFMA_SPLIT, P0K_MFMA_KERNEL, P0K_DMA_TAIL, P0K_GEMV_MF, P0K_GEMV_MQ4, P0K_GEMV_MX, P0K_GEMV_NARROW, P0K_GEMV_SN,
+ * P0K_GEMV_SLICES, P0K_GEMV_XPREP, P0K_ATTN_BQ, P0K_ATTN_SPLIT) once, when the context is created;
  * p0k_ctx_reload_env reads the switches again (no counterpart in the reference, whose tuning is gpu.tune,
  * src/core/tune.js:30-36). p0k_ctx_cus: the CU count the context plans for. */
 int p0k_ctx_reload_env(p0k_ctx *ctx);
@@ -208,19 +210,24 @@ int p0k_gemm(p0k_ctx *ctx, const p0k_gemm_args *a);            /* validate + enq
 double p0k_gemm_flops(const p0k_gemm_args *a);                 /* 2*M*N*K, the reference's return value (gemm.js:326) */
 /* p0k_gemm_noalloc: p0k_gemm that allocates nothing. No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). The
- * same kernels, with every workspace (partial sums and counters, the rms / lnmod / PixelNorm / GroupNorm X', the conv3
- * zero block) taken from one static device array per GPU, set up when the first context on that GPU is created.
- * A call needing more than p0k_gemm_noalloc_scratch_bytes() (31.5 MiB: e.g. X' of M * K * 2 bytes) is refused with
- * P0K_E_ARG. The first context that calls it on a GPU holds that GPU's array until the context is destroyed, and calls
- * from any other context on the GPU are refused with P0K_E_ARG (their stream could overlap the holder's calls). Calls
- * in order on the holder's stream do not race; each call may overwrite what the previous one left in the array.
- * Results are the same bits as p0k_gemm's. */
+ * same kernels, with every workspace (partial sums and counters, the rms / lnmod / PixelNorm / GroupNorm X', the
+ * convolutions' zero block) taken from one static device array per GPU, set up when the first context on that GPU is
+ * created. A call needing more than p0k_gemm_noalloc_scratch_bytes() (31.5 MiB: e.g. X' of M * K * 2 bytes) is refused with
+ * P0K_E_ARG, but for two that can do with less: a 2-D convolution with GroupNorm takes its image in bands (or, where not
+ * even one row of output fits, applies GroupNorm inside the register-staged kernel), and conv3 with f16 weights, PixelNorm
+ * and 96, 160, 224, ... channels applies it there too. The first context that calls it on a GPU holds that GPU's array
+ * until the context is destroyed, and calls from any other context on the GPU are refused with P0K_E_ARG (their stream
+ * could overlap the holder's calls). Calls in order on the holder's stream do not race; each call may overwrite what the
+ * previous one left in the array.
+ * Results are the same bits as p0k_gemm's outside a capture (not for q4 / q8 weights of a GroupNorm convolution that falls
+ * back to the register-staged kernel, whose order of sums differs). */
 int p0k_gemm_noalloc(p0k_ctx *ctx, const p0k_gemm_args *a);
 uint64_t p0k_gemm_noalloc_scratch_bytes(void);
 int p0k_select_tile(const p0k_gemm_args *a, p0k_tile *out);     /* the kernel and tile p0k_gemm would use on a
                                                                    256-CU device with the current environment */
 int p0k_gemm_plan(p0k_ctx *ctx, const p0k_gemm_args *a, p0k_tile *out);   /* the kernel and tile p0k_gemm uses on
                                                                    this context (its CU count and tuning switches) */
+/* (both outside a capture; neither says into how many slices K is cut. What a capture changes: see the graphs below) */
 int p0k_rowstats_check(const p0k_rowstats_args *a);
 int p0k_rowstats(p0k_ctx *ctx, const p0k_rowstats_args *a);
 
@@ -250,6 +257,11 @@ int p0k_pack_f16(const float *W, uint64_t n, uint16_t *out);
 /* ---- HIP graphs: capture the context's stream (e.g. a decode step's gemm calls), then replay it with one launch.
  *      (The reference batches dispatches into command buffers, src/core/gpu.js:203-257; a graph is the HIP form.)
  *      Between begin and end only enqueueing calls may be made (p0k_gemm, p0k_rowstats, p0k_copy).
+ *      Workspaces cannot grow during a capture, so one call of each shape should be made before it. Without it, a call that
+ *      cannot do without is refused ("must grow": rms / lnmod prompts, PixelNorm clips, decode with K split); one that
+ *      can runs by another, usually slower plan: K of a prompt unsplit, the prologue of a decode or of a GroupNorm convolution
+ *      inside its kernel. The same plans serve every such call in a capture that the caller began (there the few-queries
+ *      attention keeps one run of keys). Sums may then be in another order than outside the capture.
  *      A graph may be launched through any context. Its calls may use the workspaces of the context that captured it: a
  *      launch through another one is then ordered with that context's work (it waits for what that context has enqueued,
  *      and what that context enqueues afterwards waits for it), and refused with P0K_E_ARG while either stream is being

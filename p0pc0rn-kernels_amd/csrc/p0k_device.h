@@ -52,7 +52,7 @@ struct Params {
   uint32_t flags;
   int32_t epi;
   uint32_t tilesM, tilesN;
-  const uint8_t *Z;    // 16 zero bytes (the load-to-LDS conv3 gather reads them for padding taps)
+  const uint8_t *Z;    // zero bytes (the load-to-LDS convolutions read them for padding taps)
   uint32_t nvox;       // conv3 / conv: input voxels the call may read (frames x Hi x Wi; Hi x Wi)
   uint32_t nbase;      // load-to-LDS GEMM: first ws column of this launch (its tiles cover [nbase, N))
   float *part;         // split K: fp32 sums [slice][M][ldp] (null: one slice)

@@ -3,15 +3,15 @@
 // M0 + 16 lane / 4 lane, no registers, no LDS store instructions), weights are decoded in registers right before the
 // matrix core uses them.
 //
-// One workgroup computes a TBM x TBN tile (TBM, TBN in {128, 256}): 4 waves (2 x 2) for the smaller tiles, 8 waves
-// (2 x 4, two per SIMD, so one wave's decode and LDS reads run under the other's MFMAs) for 256 x 256 and, with f16
+// One workgroup computes a TBM x TBN tile. On large grids TBM, TBN in {128, 256}: 4 waves (2 x 2) for the smaller tiles, 8
+// waves (2 x 4, two per SIMD, so one wave's decode and LDS reads run under the other's MFMAs) for 256 x 256 and, with f16
 // or q8 weights, 256 x 128; a wave owns (TBM/2) x (TBN/2), 128 x 64 or 128 x 32 as 32x32 v_mfma_f32_32x32x16_f16
 // blocks. For grids of few or short tiles (not of convolutions), 8 waves lie 1 x 4 x 2 instead: a tile of any 32 rows x 128 columns, each wave
 // over all its rows and 32 columns, the two halves of the waves on alternate 64-k steps (WK = 2: a stage is two steps),
 // whose sums meet in LDS; and K may be cut into slices over workgroups (SPLIT), whose fp32 sums k_split_epi adds in slice
 // order before the epilogue. A weight is then decoded once per workgroup (2 x 4 decodes it in both row halves), the
 // padding rows are at most 31, and a step of a short tile does not wait for LDS four times: q4 77 x 6144 x 4096 40.3 ->
-// 26.1 us unsplit, 16.8 in 4 slices (profile: 5 us of K loop, 6 of two launches' fixed cost, 5 of partial sums).
+// 26.1 us unsplit, 16.8 in 4 slices (with the heads epilogue: 15.1 us in the slices, 4.1 in k_split_epi).
 // K moves in steps of 64 through a ring of S LDS stages:
 //   X' rows      [row][128 B], the 16-byte chunk c of row r at c ^ ((r >> 1) & 7)
 //   f16 weights  the same layout, one row per ws column
@@ -29,8 +29,11 @@
 // the decode of its weight fragments and one third of the DMA refill of the stage freed at the last barrier. One
 // barrier per step: before it, s_waitcnt vmcnt(n) leaves only the refills younger than the next stage in flight; the
 // DMA instructions are invisible to the compiler (inline asm), so every wait on them is explicit and exact.
-// After the last step the fp32 accumulators go through LDS in 128 x 128 quadrants to the shared epilogue. The K
-// order of every output element is fixed (no split-K) and independent of the tile.
+// After the last step the fp32 accumulators go through LDS, 128 x 128 or as much of the tile as fits, to the shared epilogue.
+// The order of K of an output element is the same in every tile without K halves and slices: in the convolutions, which
+// have neither (so a clip in chunks and an image in bands keep the bits of the whole), and in the column split of dma_tail.
+// Halves and slices add in a fixed order of their own, so for fp16 rows the bits depend on the plan, and with it on the
+// size of the call.
 #pragma once
 #include "p0k_device.h"
 #include "p0k_launch.h"
@@ -69,7 +72,7 @@ struct DT {
   static constexpr int STEP = A_BYTES + BC_BYTES + BS_BYTES, STAGE = WK * STEP;
   static constexpr bool TWO = NWV == 4 && WGM == 2 && 4 * STAGE <= 160 * 1024 && TBM * TBN < 256 * 256;  // two WGs per CU
   static constexpr int BUDGET = TWO ? 80 * 1024 : 160 * 1024;
-    static constexpr int SMAX = WK == 1 ? 3 : 4;
+  static constexpr int SMAX = WK == 1 ? 3 : 4;
   static constexpr int S = BUDGET / STAGE < SMAX ? BUDGET / STAGE : SMAX;
   static_assert(S >= 2, "two stages");
   // the epilogue's fp32 staging: with one workgroup per CU the whole LDS is free after the K loop, so 128 rows of the

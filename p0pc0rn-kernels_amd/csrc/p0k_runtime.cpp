@@ -65,13 +65,13 @@ struct p0k_ctx {
   uint64_t alive = 0, peak = 0, pooled = 0, hw = 0, max_buf = 0, seq = 0;
   uint64_t creates = 0, reuses = 0, evictions = 0, pooled_n = 0;
   uint64_t cap() const { return hw + max_buf; }
-  // workspace of the split-K decode GEMV: fp32 partial tiles (grown on demand) and one arrival counter per 128-column
-  // tile (zeroed once here; every call leaves them at zero again)
+  // workspace of calls whose K is split: fp32 partial sums (decode items, slices of a prompt; grown on demand) and, for the
+  // decode, one arrival counter per 128-column tile (zeroed once here; every call leaves them at zero again)
   float *ws_part = nullptr;
   uint64_t ws_part_bytes = 0;
   uint32_t *ws_cnt = nullptr;
   static constexpr uint32_t WS_COUNTERS = 1u << 16;
-  // X' of the rms / lnmod prologues for the load-to-LDS GEMM (M x K fp16, grown on demand)
+  // X' (fp16, grown on demand): the rms / lnmod rows of a GEMM or a decode, a convolution's normalised input
   void *ws_x = nullptr;
   uint64_t ws_x_bytes = 0;
   // partial rows and counters of attention over runs of keys: a fixed size, allocated with the context
@@ -83,7 +83,7 @@ struct p0k_ctx {
   unsigned long long own_capture = 0;
   // a call of the current p0k_graph_begin .. p0k_graph_end took a workspace: the graph's replays need the stream's order
   bool capture_ws = false;
-  // 256 zero bytes: the padding taps of the load-to-LDS conv3 gather read them
+  // 256 zero bytes: the padding taps of the load-to-LDS convolutions read them
   void *ws_zero = nullptr;
   // workspaces replaced by larger ones while a graph captured after their allocation may still address them: freed
   // only with the context. graph_epoch counts the graphs captured on the stream; a workspace allocated in the current
@@ -458,7 +458,8 @@ int p0k_ctx_workspace_stats(p0k_ctx *c, uint64_t *live_bytes, uint64_t *retired_
 // The allocation-free gemm (p0k_gemm_noalloc) takes every workspace from this array instead of the context's grown
 // buffers. Layout: [0, 256 KiB) one arrival counter per 128-column tile of the split decode (zero between calls:
 // the last item of a tile resets its counter), [256 KiB, +256) the zero block the conv3 gather's padding taps read,
-// [512 KiB, 32 MiB) either the split decode's fp32 partials or the rms / lnmod / PixelNorm X' of one call. Each
+// [512 KiB, 32 MiB) one call's X' (rms / lnmod rows, the PixelNorm or GroupNorm input or a band of it) and, 256-byte aligned
+// after it, its fp32 partial sums (K slices of the decode or of a prompt). Each
 // device holds its own copy; host code reaches it only through the address hipGetSymbolAddress returns for that
 // device (the array's name on the host is a stand-in, not a device address).
 static constexpr uint64_t SCRATCH_BYTES = 32ull << 20, SCRATCH_CNT = 0, SCRATCH_ZERO = 256ull << 10,
@@ -508,7 +509,7 @@ struct WsSource {
       if (need > SCRATCH_BYTES - SCRATCH_WS - xoff)
         return set_err(P0K_E_ARG, "gemm_noalloc: the split decode needs " + std::to_string(need) +
                                       " bytes of partials, the scratch array holds " +
-                                      std::to_string(SCRATCH_BYTES - SCRATCH_WS));
+                                      std::to_string(SCRATCH_BYTES - SCRATCH_WS - xoff) + " beside the call's X'");
       *out = (float *)(scratch + SCRATCH_WS + xoff);
       return P0K_OK;
     }
@@ -595,7 +596,8 @@ struct WsSource {
 // 2-D convolution with GroupNorm + SiLU on the load-to-LDS kernel: they are applied once per input element into the X'
 // workspace, and the gather reads plain fp16 pixels (the register-staged kernel applies them once per tap and column
 // tile). A workspace smaller than the image takes it in bands of output rows, each with the input rows that its taps
-// touch (the K order, and so the bits, do not change); without room for one output row, the register-staged kernel.
+// touch; without room for one output row, or for any in a capture, the register-staged kernel. The bits are the same in every
+// case with f16 weights; with q4 / q8 weights the register-staged kernel has another order of k inside a 64-k step.
 static hipError_t conv_gn(const p0k::Params &p0, const p0k::Plan &plan, const p0k::DmaPlan &d, const p0k::Tuning &tune, WsSource &ws,
                           int *err) {
   p0k::Params p = p0;
