@@ -503,48 +503,50 @@ struct WsSource {
   p0k_ctx *c;
   uint8_t *scratch;   // non-null: the allocation-free path
   uint64_t xoff = 0;  // and the bytes of X' at its start, beside which the partial sums lie
+  template <class T>
+  T *taken(T *ws) {   // a graph being captured holds it (p0k_graph_launch)
+    if (ws) c->capture_ws = true;
+    return ws;
+  }
   int part(uint64_t need, float **out) {
-    c->capture_ws = true;
     if (scratch) {
       if (need > SCRATCH_BYTES - SCRATCH_WS - xoff)
         return set_err(P0K_E_ARG, "gemm_noalloc: the split decode needs " + std::to_string(need) +
                                       " bytes of partials, the scratch array holds " +
                                       std::to_string(SCRATCH_BYTES - SCRATCH_WS - xoff) + " beside the call's X'");
-      *out = (float *)(scratch + SCRATCH_WS + xoff);
+      *out = taken((float *)(scratch + SCRATCH_WS + xoff));
       return P0K_OK;
     }
     if (int r = grow_ws(c, (void **)&c->ws_part, &c->ws_part_bytes, &c->ws_part_epoch, need, "decode")) return r;
-    *out = c->ws_part;
+    *out = taken(c->ws_part);
     return P0K_OK;
   }
   int xws(uint64_t need, void **out) {
-    c->capture_ws = true;
     if (scratch) {
       if (need > SCRATCH_BYTES - SCRATCH_WS)
         return set_err(P0K_E_ARG, "gemm_noalloc: the prologue needs " + std::to_string(need) +
                                       " bytes of X', the scratch array holds " + std::to_string(SCRATCH_BYTES - SCRATCH_WS));
-      *out = scratch + SCRATCH_WS;
+      *out = taken(scratch + SCRATCH_WS);
       return P0K_OK;
     }
     if (int r = grow_ws(c, &c->ws_x, &c->ws_x_bytes, &c->ws_x_epoch, need, "prologue")) return r;
-    *out = c->ws_x;
+    *out = taken(c->ws_x);
     return P0K_OK;
   }
   // partial sums of a GEMM over slices of K, beside `xbytes` of X': null where the call has to do without (as xws_if;
   // the planner keeps both inside the scratch array)
   int slices_if(uint64_t xbytes, uint64_t need, float **out) {
     *out = nullptr;
-    c->capture_ws = true;
     if (scratch) {
       xbytes = (xbytes + 255) / 256 * 256;
-      if (xbytes + need <= SCRATCH_BYTES - SCRATCH_WS) *out = (float *)(scratch + SCRATCH_WS + xbytes);
+      if (xbytes + need <= SCRATCH_BYTES - SCRATCH_WS) *out = taken((float *)(scratch + SCRATCH_WS + xbytes));
       return P0K_OK;
     }
     bool capturing, ok;
     if (int rr = ws_allowed(c, &capturing, &ok)) return rr;
     if (!ok || (capturing && need > c->ws_part_bytes)) return P0K_OK;
     const int r = grow_ws(c, (void **)&c->ws_part, &c->ws_part_bytes, &c->ws_part_epoch, need, "split");
-    if (r == P0K_OK) *out = c->ws_part;
+    if (r == P0K_OK) *out = taken(c->ws_part);
     if (r != P0K_E_NOMEM) return r;
     (void)hipGetLastError();
     return P0K_OK;
@@ -566,9 +568,8 @@ struct WsSource {
   int xws_if(uint64_t need, void **out, uint64_t *have) {
     *out = nullptr;
     *have = 0;
-    c->capture_ws = true;
     if (scratch) {
-      *out = scratch + SCRATCH_WS;
+      *out = taken(scratch + SCRATCH_WS);
       *have = std::min<uint64_t>(need, SCRATCH_BYTES - SCRATCH_WS);
       return P0K_OK;
     }
@@ -576,13 +577,13 @@ struct WsSource {
     if (int rr = ws_allowed(c, &capturing, &ok)) return rr;
     if (!ok) return P0K_OK;
     if (capturing && need > c->ws_x_bytes) {
-      *out = c->ws_x;
+      *out = taken(c->ws_x);
       *have = c->ws_x_bytes;
       return P0K_OK;
     }
     const int r = grow_ws(c, &c->ws_x, &c->ws_x_bytes, &c->ws_x_epoch, need, "prologue");
     if (r == P0K_OK) {
-      *out = c->ws_x;
+      *out = taken(c->ws_x);
       *have = need;
     }
     if (r != P0K_E_NOMEM) return r;

@@ -148,3 +148,30 @@ def test_capture_ended_by_the_caller_is_forgotten():
         assert np.array_equal(captured(), one)
     finally:
         dev.close()
+
+
+def test_graph_without_workspaces_is_launched_freely():
+    """A graph none of whose calls took a workspace (a prompt captured before the workspace for its slices of K was there
+    among them) has no order to keep: another context launches it also while the first is being captured."""
+    own, other = p0k.Device(0), p0k.Device(0)
+    print("[p0k-test] graph without workspaces", flush=True)
+    try:
+        cs = [make_case(enc="q4g32a.t64", epi="f16", M=M, N=512, K=4096, wscale=0.02, seed=47) for M in (1, 77)]
+        ds = [{k: own.upload(v) for k, v in c.bufs.items()} for c in cs]
+        own.graph_begin()
+        for c, d in zip(cs, ds):
+            own.gemm(c.args(lambda n: d[n]))
+        g = own.graph_end()
+        own.graph_begin()
+        other.graph_launch(g)
+        own.graph_destroy(own.graph_end())
+        other.done()
+        for c, d in zip(cs, ds):
+            got, size = own.read(d["y"], np.uint16, c.bufs["y"].size), c.bufs["y"].size
+            own.upload(np.zeros(size, np.uint16), d["y"])
+            own.graph_launch(g)
+            assert got.any() and np.array_equal(own.read(d["y"], np.uint16, size), got)
+        own.graph_destroy(g)
+    finally:
+        own.close()
+        other.close()
